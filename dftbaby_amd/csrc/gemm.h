@@ -15,6 +15,8 @@ struct GemmTimer {
   void end(hipStream_t st, int cls, double flops);
 };
 int gemm_bf16x3_launch(const GemmArgs& p, hipStream_t st);
+// *big = 1 when the 128 x 128 workgroup tile was taken
+int gemm_f64_launch(const GemmArgs& p, hipStream_t st, int* big);
 int gemm_reduce_launch(const double* P, long sP, int nsplit, double* C, long n, double alpha, double beta,
                        hipStream_t st);
 

@@ -1,17 +1,17 @@
-// Batched, strided MFMA GEMM for gfx950 (FP64 and FP32 operands).
+// Batched, strided GEMM entry point for gfx950, and its FP32 kernel.
 //
 //   C[b] (+)= alpha * op(A[b]) * op(B[b]) + beta * C[b]
 //
 // It carries every dense contraction of the Casida matvec and of the
 // Davidson loop: the gamma-fold of the transition charges, the "expand"
 // and "contract" halves of the two long-range exchange terms, the Coulomb
-// projections, Gram matrices and subspace linear combinations.
+// projections, Gram matrices and subspace linear combinations.  FP64 operands go
+// to gemm_f64.hip, BF16x3 pairs to gemm_bf16.hip.
 //
-// Tiling: 256 threads = 4 wave64s in a 2x2 arrangement; each wave owns a
-// (BM/2)x(BN/2) block of 16x16 MFMA tiles (v_mfma_f64_16x16x4f64 /
-// v_mfma_f32_16x16x4f32).  Operand tiles are staged K-major in LDS
-// (double buffered, one barrier per K step) so that the 16 lanes that feed
-// one MFMA row/column read 16 consecutive LDS words.
+// FP32 tiling: 256 threads = 4 wave64s in a 2x2 arrangement; each wave owns a
+// (BM/2)x(BN/2) block of 16x16 MFMA tiles (v_mfma_f32_16x16x4f32).  Operand tiles
+// are staged K-major in LDS (double buffered, one barrier per K step) so that the
+// 16 lanes that feed one MFMA row/column read 16 consecutive LDS words.
 //
 // Output modes: plain row-major, or a column and/or row remap where output
 // column n is split as (n / cdiv, n % cdiv) and written at (n / cdiv) * cstr +
@@ -21,19 +21,6 @@
 // per-slice partial results at C + slice * sCk (reduced by gemm_reduce).
 #include "common.h"
 #include "gemm.h"
-
-template <typename T> struct IsF64 { static constexpr bool value = false; };
-template <> struct IsF64<double> { static constexpr bool value = true; };
-template <typename T> struct AccT;
-template <> struct AccT<double> { typedef d4_t type; };
-template <> struct AccT<float> { typedef f4_t type; };
-
-__device__ __forceinline__ d4_t mfma16(double a, double b, d4_t c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ f4_t mfma16(float a, float b, f4_t c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
 
 __device__ __forceinline__ void store_out(const GemmArgs& p, long off, double val) {
   if (p.out_type == GEMM_OUT_F64) {
@@ -53,11 +40,11 @@ __device__ __forceinline__ void store_out(const GemmArgs& p, long off, double va
   }
 }
 
-// WGM x (4 / WGM) waves over the BM x BN tile (2 x 2 for the square tiles; 1 x 4
-// and 4 x 1 for the 32- and 48-wide tiles of the tall-skinny basis products).
-template <typename T, int BM, int BN, int BK, bool AT, bool BT, int WGM = 2>
-__global__ __launch_bounds__(256) void gemm_fp_kernel(GemmArgs p) {
-  typedef typename AccT<T>::type V4;
+// WGM x (4 / WGM) waves over the BM x BN tile (2 x 2 for the square tiles; 1 x 4 for
+// the 16- to 48-row tiles of the Coulomb products of vector blocks).
+template <int BM, int BN, int BK, bool AT, bool BT, int WGM = 2>
+__global__ __launch_bounds__(256) void gemm_f32_kernel(GemmArgs p) {
+  typedef float T;
   __shared__ T As[2][BK][BM + 1];
   __shared__ T Bs[2][BK][BN + 1];
   constexpr int WGN = 4 / WGM;
@@ -120,11 +107,11 @@ __global__ __launch_bounds__(256) void gemm_fp_kernel(GemmArgs p) {
     }
   };
 
-  V4 acc[TM][TN];
+  f4_t acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = (V4)(0);
+    for (int j = 0; j < TN; ++j) acc[i][j] = (f4_t)(0.0f);
 
   const long nk = (kend > kbeg) ? (kend - kbeg + BK - 1) / BK : 0;
   if (nk > 0) {
@@ -145,7 +132,7 @@ __global__ __launch_bounds__(256) void gemm_fp_kernel(GemmArgs p) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(af[i], bf[j], acc[i][j]);
+          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i], bf[j], acc[i][j], 0, 0, 0);
       }
       if (kt + 1 < nk) sstore(cur ^ 1);
       __syncthreads();
@@ -167,10 +154,8 @@ __global__ __launch_bounds__(256) void gemm_fp_kernel(GemmArgs p) {
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      // accumulator row: v_mfma_f64_16x16x4f64 holds rows (lane/16) + 4r,
-      // v_mfma_f32_16x16x4f32 rows 4(lane/16) + r (both: column lane%16)
-      const int rr = IsF64<T>::value ? ((lane >> 4) + 4 * r) : (4 * (lane >> 4) + r);
-      const long row = m0 + wm * WBM + i * 16 + rr;
+      // v_mfma_f32_16x16x4f32 holds accumulator rows 4(lane/16) + r, column lane%16
+      const long row = m0 + wm * WBM + i * 16 + 4 * (lane >> 4) + r;
       if (row >= M) continue;
       const long ro = cbase + gemm_row_part(p, row);
       const long hr = had_on ? gemm_had_row(p, row) : 0;
@@ -194,13 +179,13 @@ __global__ void gemm_reduce_kernel(const double* P, long sP, int nsplit, double*
   C[i] = s;
 }
 
-template <typename T, int BM, int BN, int BK, int WGM = 2>
-static void launch_fp(const GemmArgs& p, hipStream_t st) {
+template <int BM, int BN, int BK, int WGM = 2>
+static void launch_f32(const GemmArgs& p, hipStream_t st) {
   dim3 grid(ceil_div(p.N, BN), ceil_div(p.M, BM), p.batch * p.ksplit);
-  if (!p.a_trans && !p.b_trans) hipLaunchKernelGGL((gemm_fp_kernel<T, BM, BN, BK, false, false, WGM>), grid, dim3(256), 0, st, p);
-  else if (p.a_trans && !p.b_trans) hipLaunchKernelGGL((gemm_fp_kernel<T, BM, BN, BK, true, false, WGM>), grid, dim3(256), 0, st, p);
-  else if (!p.a_trans && p.b_trans) hipLaunchKernelGGL((gemm_fp_kernel<T, BM, BN, BK, false, true, WGM>), grid, dim3(256), 0, st, p);
-  else hipLaunchKernelGGL((gemm_fp_kernel<T, BM, BN, BK, true, true, WGM>), grid, dim3(256), 0, st, p);
+  if (!p.a_trans && !p.b_trans) hipLaunchKernelGGL((gemm_f32_kernel<BM, BN, BK, false, false, WGM>), grid, dim3(256), 0, st, p);
+  else if (p.a_trans && !p.b_trans) hipLaunchKernelGGL((gemm_f32_kernel<BM, BN, BK, true, false, WGM>), grid, dim3(256), 0, st, p);
+  else if (!p.a_trans && p.b_trans) hipLaunchKernelGGL((gemm_f32_kernel<BM, BN, BK, false, true, WGM>), grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL((gemm_f32_kernel<BM, BN, BK, true, true, WGM>), grid, dim3(256), 0, st, p);
 }
 
 // ---------------------------------------------------------------------------
@@ -285,31 +270,22 @@ int gemm_launch(const GemmArgs& p0, hipStream_t st, bool timed) {
   GemmTimer tm;
   tm.slot = -1;
   if (timed) tm.begin(st);
+  int big64 = 0;
   if (p.in_type == GEMM_IN_F64) {
-    // tall-skinny products of the Davidson basis (one side 20-40 vectors, the other
-    // hundreds of basis vectors or the pair index): narrow tiles cut the padded
-    // MFMA work, which bounds these calls at the FP64 MFMA rate
-    if (small && p.M <= 16 && p.N > 48) launch_fp<double, 16, 64, 16, 1>(p, st);
-    else if (small && p.M <= 32 && p.N > 48) launch_fp<double, 32, 64, 16, 1>(p, st);
-    else if (small && p.M <= 48 && p.N > 48) launch_fp<double, 48, 64, 16, 1>(p, st);
-    else if (small && p.N <= 32 && p.M > 48) launch_fp<double, 64, 32, 16, 4>(p, st);
-    else if (small && p.N <= 48 && p.M > 48) launch_fp<double, 64, 48, 16, 4>(p, st);
-    else if (small && p.N <= 80 && p.M > 80) launch_fp<double, 64, 80, 16, 4>(p, st);   // both Gram halves of a block
-    else if (small && p.M <= 48 && p.N <= 48 && p.M > 32) launch_fp<double, 48, 64, 16, 1>(p, st);  // a block's own Gram
-    else if (small) launch_fp<double, 64, 64, 16>(p, st);
-    else launch_fp<double, 128, 128, 16>(p, st);
+    const int rc = gemm_f64_launch(p, st, &big64);
+    if (rc) return rc;
   } else {
     // the Coulomb projection / expansion of a vector block: M = block size (<= 48 rows
     // per tile instead of 64 cuts the padded MFMA work by a quarter)
-    if (small && p.M <= 48 && p.M > 32 && p.N >= 4096) launch_fp<float, 48, 128, 32, 1>(p, st);
-    else if (small && p.M <= 48 && p.M > 32) launch_fp<float, 48, 64, 32, 1>(p, st);
-    else if (small && p.M <= 16) launch_fp<float, 16, 64, 32, 1>(p, st);
-    else if (small && p.M <= 32) launch_fp<float, 32, 64, 32, 1>(p, st);
-    else if (small) launch_fp<float, 64, 64, 32>(p, st);
-    else launch_fp<float, 128, 128, 32>(p, st);
+    if (small && p.M <= 48 && p.M > 32 && p.N >= 4096) launch_f32<48, 128, 32, 1>(p, st);
+    else if (small && p.M <= 48 && p.M > 32) launch_f32<48, 64, 32, 1>(p, st);
+    else if (small && p.M <= 16) launch_f32<16, 64, 32, 1>(p, st);
+    else if (small && p.M <= 32) launch_f32<32, 64, 32, 1>(p, st);
+    else if (small) launch_f32<64, 64, 32>(p, st);
+    else launch_f32<128, 128, 32>(p, st);
   }
   const int cls = p.in_type == GEMM_IN_F64
-                      ? (small ? GT_F64_64 : ((p.a_trans || p.b_trans) ? GT_F64_128_T : GT_F64_128))
+                      ? (!big64 ? GT_F64_64 : ((p.a_trans || p.b_trans) ? GT_F64_128_T : GT_F64_128))
                       : (small ? GT_F32_64 : GT_F32_128);
   tm.end(st, cls, 2.0 * p.M * p.N * (double)p.K * p.batch);
   DFTB_CHECK_LAUNCH();
