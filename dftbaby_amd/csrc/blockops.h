@@ -26,8 +26,34 @@ __host__ __device__ static EigLayout eig_layout(int l, int nev) {
 }
 
 
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, hi, CTRL, 0xf, 0xf, true),
+                          __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xf, 0xf, true));
+}
+
+// Sum over the wave in every lane: the butterfly v_i + v_{i ^ o}, o = 32, 16, .. 1.  The
+// partners come through v_permlane swaps and row rotations (after the step o = 8 a row's
+// halves agree, so that a rotation by o reads the same value as lane i ^ o) instead of
+// ds_bpermute: 6 steps of ~25 cycles instead of ~120.
 __device__ __forceinline__ double wave_sum(double v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  {
+    const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+    const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    v = __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+  }
+  {
+    const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+    const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    v = __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+  }
+  v += dpp_f64<0x128>(v);   // row_ror:8
+  v += dpp_f64<0x124>(v);   // row_ror:4
+  v += dpp_f64<0x122>(v);   // row_ror:2
+  v += dpp_f64<0x121>(v);   // row_ror:1
   return v;
 }
 
@@ -42,6 +68,18 @@ __device__ double blk_sum(double v, double* sh) {
   return s;
 }
 
+// maximum over the workgroup (all threads get it)
+__device__ double blk_max_any(double v, double* sh) {
+  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  __syncthreads();
+  if (lane == 0) sh[wv] = v;
+  __syncthreads();
+  double m = sh[0];
+  for (int i = 1; i < (int)(blockDim.x >> 6); ++i) m = fmax(m, sh[i]);
+  return m;
+}
+
 // Sturm count: number of eigenvalues of the tridiagonal (d, e) below x.
 typedef __attribute__((address_space(3))) double lds_f64;
 typedef __attribute__((address_space(3))) int lds_i32;
@@ -52,6 +90,7 @@ __device__ int sturm_count(const lds_f64* d, const lds_f64* e, int l, double x, 
   double q = d[0] - x;
   if (fabs(q) < pivmin) q = -pivmin;
   if (q < 0) ++c;
+#pragma unroll 8
   for (int i = 1; i < l; ++i) {
     q = d[i] - x - e[i - 1] * e[i - 1] / q;
     if (fabs(q) < pivmin) q = -pivmin;
@@ -158,18 +197,179 @@ __device__ void tri_apply(int l, const D* __restrict__ u0r, const D* __restrict_
 }
 
 
+// ---- inverse iteration of one eigenvalue cluster by one wavefront -------------------
+// The recurrences (substitution, dot products, norms) are chains over the vector's
+// entries: lane 0 runs them on operands in LDS, unrolled so that the reads run ahead of
+// the chain.  What is not a chain (updates, scaling, loads, stores) is spread over the
+// lanes.  The factors arrive in blocks of 64 steps, one step per lane, the next block's
+// loads issued before the current block's steps.  One thread per cluster on global memory
+// paid a memory latency per entry and serialised the clusters of a wave: the kernel took
+// 17.7 ms for 20 roots at l = 620, this form takes 4.8 ms (same results).
+#define EIG_STAGE 320            // LDS doubles per wave: five arrays of 64
+#define EIG_STAGE_WAVES 8
+
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// one forward step: entry x_k leaves as `keep`, the eliminated next entry stays in c
+__device__ __forceinline__ double tri_forward(double& c, double nx, double m, int pv) {
+  const double keep = pv ? nx : c;
+  c = pv ? c - m * nx : nx - m * c;
+  return keep;
+}
+
+// x <- (T - lam I)^{-1} x with the factors of tri_factor, x (l doubles) and stg in LDS
+__device__ void tri_apply_wave(int l, const double* __restrict__ u0r, const double* __restrict__ u1,
+                               const double* __restrict__ u2, const double* __restrict__ mlt,
+                               const int* __restrict__ piv, lds_f64* x, lds_f64* stg) {
+  const int lane = threadIdx.x & 63;
+  lds_f64 *sm = stg, *s0 = stg, *s1 = stg + 64, *s2 = stg + 128;
+  double c = x[0];
+  const int nf = l - 1;                      // forward steps
+  double gm = 0.0;
+  int gp = 0;
+  if (lane < nf) { gm = mlt[lane]; gp = piv[lane]; }
+  for (int kb = 0; kb < nf; kb += 64) {
+    const int n = nf - kb < 64 ? nf - kb : 64;
+    sm[lane] = gm;
+    const unsigned long long pm = __ballot(gp != 0);
+    wave_lds_fence();
+    if (kb + 64 + lane < nf) { gm = mlt[kb + 64 + lane]; gp = piv[kb + 64 + lane]; }
+    lds_f64* xb = x + kb;
+    if (lane == 0) {
+      int h = 0;
+      for (; h + 16 <= n; h += 16) {
+        double nx[16], m[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) { nx[u] = xb[h + u + 1]; m[u] = sm[h + u]; }
+#pragma unroll
+        for (int u = 0; u < 16; ++u) xb[h + u] = tri_forward(c, nx[u], m[u], (int)(pm >> (h + u)) & 1);
+      }
+      for (; h < n; ++h) xb[h] = tri_forward(c, xb[h + 1], sm[h], (int)(pm >> h) & 1);
+    }
+    wave_lds_fence();
+  }
+  if (lane == 0) x[l - 1] = c;
+  wave_lds_fence();
+  // backward: step t handles entry l - 1 - t
+  double g0 = 0.0, g1 = 0.0, g2 = 0.0;
+  if (lane < l) { g0 = u0r[l - 1 - lane]; g1 = u1[l - 1 - lane]; g2 = u2[l - 1 - lane]; }
+  double x1 = 0.0, x2 = 0.0;
+  for (int kb = 0; kb < l; kb += 64) {
+    const int n = l - kb < 64 ? l - kb : 64;
+    s0[lane] = g0;
+    s1[lane] = g1;
+    s2[lane] = g2;
+    wave_lds_fence();
+    if (kb + 64 + lane < l) {
+      g0 = u0r[l - 65 - kb - lane];
+      g1 = u1[l - 65 - kb - lane];
+      g2 = u2[l - 65 - kb - lane];
+    }
+    lds_f64* xb = x + (l - 1 - kb);
+    if (lane == 0) {
+      int h = 0;
+      for (; h + 16 <= n; h += 16) {
+        double xv[16], a1[16], a2[16], r0[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+          xv[u] = xb[-(h + u)];
+          a1[u] = s1[h + u];
+          a2[u] = s2[h + u];
+          r0[u] = s0[h + u];
+        }
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+          const double sv = (xv[u] - a1[u] * x1 - a2[u] * x2) * r0[u];
+          xb[-(h + u)] = sv;
+          x2 = x1;
+          x1 = sv;
+        }
+      }
+      for (; h < n; ++h) {
+        const double sv = (xb[-h] - s1[h] * x1 - s2[h] * x2) * s0[h];
+        xb[-h] = sv;
+        x2 = x1;
+        x1 = sv;
+      }
+    }
+    wave_lds_fence();
+  }
+}
+
+// sum_i a_i x_i as one chain over i (a: global with stride lda, or x itself when null); the
+// result in every lane
+__device__ double dot_chain_wave(int l, const double* __restrict__ a, long lda, const lds_f64* x, lds_f64* stg) {
+  const int lane = threadIdx.x & 63;
+  double s = 0.0;
+  double g = (a && lane < l) ? a[lane * lda] : 0.0;
+  for (int kb = 0; kb < l; kb += 64) {
+    const int n = l - kb < 64 ? l - kb : 64;
+    const lds_f64 *xb = x + kb, *y = xb;
+    if (a) {
+      stg[lane] = g;
+      wave_lds_fence();
+      y = stg;
+      if (kb + 64 + lane < l) g = a[(kb + 64 + lane) * lda];
+    }
+    if (lane == 0) {
+      int h = 0;
+      for (; h + 16 <= n; h += 16) {
+        double p[16], q[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) { p[u] = y[h + u]; q[u] = xb[h + u]; }
+#pragma unroll
+        for (int u = 0; u < 16; ++u) s += p[u] * q[u];
+      }
+      for (; h < n; ++h) s += y[h] * xb[h];
+    }
+    wave_lds_fence();
+  }
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(s)),
+                          __builtin_amdgcn_readfirstlane(__double2loint(s)));
+}
+
+// members m0 .. m1 - 1 of one cluster (factors of member m at scr + 6 l m) into Z
+__device__ void cluster_wave(int l, int nev, int m0, int m1, const double* __restrict__ scr, double* __restrict__ Z,
+                             lds_f64* x, lds_f64* stg) {
+  const int lane = threadIdx.x & 63;
+  for (int m = m0; m < m1; ++m) {
+    const double* base = scr + (size_t)6 * l * m;
+    for (int i = lane; i < l; i += 64) x[i] = hash_unit((unsigned)m, (unsigned)i);
+    wave_lds_fence();
+    for (int it = 0; it < 4; ++it) {
+      tri_apply_wave(l, base, base + l, base + 2 * l, base + 3 * l, (const int*)(base + 4 * l), x, stg);
+      for (int mm = m0; mm < m; ++mm) {
+        const double s = dot_chain_wave(l, Z + mm, nev, x, stg);
+        for (int i = lane; i < l; i += 64) x[i] -= s * Z[(long)i * nev + mm];
+        wave_lds_fence();
+      }
+      double nrm = sqrt(dot_chain_wave(l, nullptr, 0, x, stg));
+      if (!(nrm > 0.0)) nrm = 1.0;
+      for (int i = lane; i < l; i += 64) x[i] /= nrm;
+      wave_lds_fence();
+    }
+    for (int i = lane; i < l; i += 64) Z[(long)i * nev + m] = x[i];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");   // later members read it from global memory
+    wave_lds_fence();
+  }
+}
+
 // Lowest nev eigenpairs of the symmetric l x l matrix A (leading dim ld), one
 // workgroup: Householder tridiagonalisation, Sturm bisection, inverse
 // iteration (clusters re-orthogonalised), back-transformation.  sv, sp: LDS
-// scratch of cap >= l doubles each; sh: >= blockDim/64 doubles; s_bnd: 2.
+// scratch of cap >= l doubles each; sh: >= blockDim/64 doubles; s_bnd: 2; stg:
+// EIG_STAGE_WAVES * EIG_STAGE doubles of LDS.
 __device__ __noinline__ void syevx_tail(int l, int nev, double* __restrict__ evals, double* __restrict__ evecs,
                                         char* __restrict__ ws, int* __restrict__ info, double* sv, double* sp,
-                                        double* sh, double* s_bnd, int cap);
+                                        double* sh, double* s_bnd, int cap, double* stg);
 
 __device__ __noinline__ void syevx_block(const double* __restrict__ A, int l, int ld, int nev,
                                          double* __restrict__ evals, double* __restrict__ evecs,
                                          char* __restrict__ ws, int* __restrict__ info, double* sv, double* sp,
-                                         double* sh, double* s_bnd, int cap) {
+                                         double* sh, double* s_bnd, int cap, double* stg) {
   EigLayout Lo = eig_layout(l, nev);
   double* W = (double*)(ws + Lo.W);
   double* d = (double*)(ws + Lo.d);
@@ -231,7 +431,7 @@ __device__ __noinline__ void syevx_block(const double* __restrict__ A, int l, in
     for (int r = tid; r < n2; r += blockDim.x) W[(long)(j + 1 + r) * l + j] = sv[r];
     __syncthreads();
   }
-  syevx_tail(l, nev, evals, evecs, ws, info, sv, sp, sh, s_bnd, cap);
+  syevx_tail(l, nev, evals, evecs, ws, info, sv, sp, sh, s_bnd, cap, stg);
 }
 
 // Steps after the Householder reduction of W (reflectors below the first
@@ -240,7 +440,7 @@ __device__ __noinline__ void syevx_block(const double* __restrict__ A, int l, in
 // sv, sp: LDS scratch of cap >= l doubles each (they hold d and e).
 __device__ __noinline__ void syevx_tridiag_vectors(int l, int nev, double* __restrict__ evals,
                                                    char* __restrict__ ws, double* sv, double* sp, double* sh,
-                                                   double* s_bnd, int cap) {
+                                                   double* s_bnd, int cap, double* stg) {
   EigLayout Lo = eig_layout(l, nev);
   double* W = (double*)(ws + Lo.W);
   double* d = (double*)(ws + Lo.d);
@@ -255,20 +455,30 @@ __device__ __noinline__ void syevx_tridiag_vectors(int l, int nev, double* __res
     }
     d[l - 1] = W[(long)(l - 1) * l + (l - 1)];
     if (l >= 1) e[l - 1] = 0.0;
-    // Gershgorin bounds
-    double lo = 1e300, hi = -1e300;
-    for (int i = 0; i < l; ++i) {
-      double r = (i > 0 ? fabs(e[i - 1]) : 0.0) + (i < l - 1 ? fabs(e[i]) : 0.0);
-      lo = fmin(lo, d[i] - r);
-      hi = fmax(hi, d[i] + r);
-    }
-    s_bnd[0] = lo;
-    s_bnd[1] = hi;
   }
   __syncthreads();
   for (int i = tid; i < l; i += blockDim.x) {
     sv[i] = d[i];
     sp[i] = e[i];
+  }
+  __syncthreads();
+  // Gershgorin bounds and the largest e^2 (minima and maxima: any order)
+  double emax2 = 0.0;
+  {
+    double lo = 1e300, hi = -1e300;
+    for (int i = tid; i < l; i += blockDim.x) {
+      const double r = (i > 0 ? fabs(sp[i - 1]) : 0.0) + (i < l - 1 ? fabs(sp[i]) : 0.0);
+      lo = fmin(lo, sv[i] - r);
+      hi = fmax(hi, sv[i] + r);
+      if (i + 1 < l) emax2 = fmax(emax2, sp[i] * sp[i]);
+    }
+    lo = -blk_max_any(-lo, sh);
+    hi = blk_max_any(hi, sh);
+    emax2 = blk_max_any(emax2, sh);
+    if (tid == 0) {
+      s_bnd[0] = lo;
+      s_bnd[1] = hi;
+    }
   }
   __syncthreads();
   const double* dl = sv;
@@ -277,8 +487,6 @@ __device__ __noinline__ void syevx_tridiag_vectors(int l, int nev, double* __res
   const lds_f64* lel = (const lds_f64*)sp;
   const double lo0 = s_bnd[0], hi0 = s_bnd[1];
   const double tnorm = fmax(fabs(lo0), fabs(hi0));
-  double emax2 = 0.0;
-  for (int i = 0; i + 1 < l; ++i) emax2 = fmax(emax2, el[i] * el[i]);
   const double pivmin = 2.2250738585072014e-308 * fmax(1.0, emax2);
   const double eps = 1.1102230246251565e-16;
 
@@ -348,7 +556,7 @@ __device__ __noinline__ void syevx_tridiag_vectors(int l, int nev, double* __res
   __syncthreads();
 
   // ---- 3. inverse iteration.  Clusters (gap < 1e-3 ||T||) of at most EIG_SMALL_CLUSTER
-  // members are handled by the thread owning their first member; larger clusters
+  // members are handled by one wave each; larger clusters
   // are processed by the whole workgroup with classical Gram-Schmidt (twice)
   // against the earlier members in every iteration.  Member m of a cluster
   // starting at m0 uses the shift evals[m] + 10 (m - m0) eps ||T||; its LU
@@ -365,36 +573,29 @@ __device__ __noinline__ void syevx_tridiag_vectors(int l, int nev, double* __res
     tri_factor(dl, el, l, lam, tiny, base, base + l, base + 2 * l, base + 3 * l, (int*)(base + 4 * l));
   }
   __syncthreads();
-  for (int m0 = tid; m0 < nev; m0 += blockDim.x) {
-    if (m0 > 0 && evals[m0] - evals[m0 - 1] < ortol) continue;  // not a cluster head
-    int m1 = m0 + 1;
-    while (m1 < nev && evals[m1] - evals[m1 - 1] < ortol) ++m1;
-    if (m1 - m0 > EIG_SMALL_CLUSTER) continue;
-    for (int m = m0; m < m1; ++m) {
-      double* base = scr + (size_t)6 * l * m;
-      double* x = base + 5 * l;
-      for (int i = 0; i < l; ++i) x[i] = hash_unit((unsigned)m, (unsigned)i);
-      for (int it = 0; it < 4; ++it) {
-        tri_apply(l, base, base + l, base + 2 * l, base + 3 * l, (const int*)(base + 4 * l), x);
-        for (int mm = m0; mm < m; ++mm) {
-          double s = 0.0;
-          for (int i = 0; i < l; ++i) s += Z[(long)i * nev + mm] * x[i];
-          for (int i = 0; i < l; ++i) x[i] -= s * Z[(long)i * nev + mm];
-        }
-        double nrm = 0.0;
-        for (int i = 0; i < l; ++i) nrm += x[i] * x[i];
-        nrm = sqrt(nrm);
-        if (!(nrm > 0.0)) nrm = 1.0;
-        for (int i = 0; i < l; ++i) x[i] /= nrm;
+  const int lane = tid & 63, wv = tid >> 6, nw = blockDim.x >> 6;
+  {
+    // one wave per cluster; the iterates live in sv / sp (d and e are used up), so at
+    // most 2 floor(cap / l) waves take part
+    int nwl = 2 * (cap / l);
+    if (nwl > nw) nwl = nw;
+    if (nwl > EIG_STAGE_WAVES) nwl = EIG_STAGE_WAVES;
+    if (wv < nwl) {
+      lds_f64* x = (lds_f64*)((wv & 1 ? sp : sv) + (size_t)(wv >> 1) * l);
+      lds_f64* st = (lds_f64*)(stg + wv * EIG_STAGE);
+      int at = 0;                              // small clusters in order, dealt to the waves
+      for (int m0 = 0; m0 < nev;) {
+        int m1 = m0 + 1;
+        while (m1 < nev && evals[m1] - evals[m1 - 1] < ortol) ++m1;
+        if (m1 - m0 <= EIG_SMALL_CLUSTER && at++ % nwl == wv) cluster_wave(l, nev, m0, m1, scr, Z, x, st);
+        m0 = m1;
       }
-      for (int i = 0; i < l; ++i) Z[(long)i * nev + m] = x[i];
     }
   }
   __syncthreads();
   // large clusters, cooperatively.  The member's factors and iterate are staged in
   // the LDS buffers (free once the factors exist) when 4 l doubles fit, so the
   // serial solve runs on LDS; the Gram-Schmidt coefficients take one wave each.
-  const int lane = tid & 63, wv = tid >> 6, nw = blockDim.x >> 6;
   const bool stage = 4 * l <= cap;
   for (int m0 = 0; m0 < nev;) {
     int m1 = m0 + 1;
@@ -487,7 +688,7 @@ __device__ __noinline__ void syevx_back_block(int l, int nev, double* __restrict
 
 __device__ __noinline__ void syevx_tail(int l, int nev, double* __restrict__ evals, double* __restrict__ evecs,
                                         char* __restrict__ ws, int* __restrict__ info, double* sv, double* sp,
-                                        double* sh, double* s_bnd, int cap) {
-  syevx_tridiag_vectors(l, nev, evals, ws, sv, sp, sh, s_bnd, cap);
+                                        double* sh, double* s_bnd, int cap, double* stg) {
+  syevx_tridiag_vectors(l, nev, evals, ws, sv, sp, sh, s_bnd, cap, stg);
   syevx_back_block(l, nev, evecs, ws, sv);
 }

@@ -4,8 +4,7 @@
 // (scipy.linalg.sqrtm + numpy.linalg.eigh, DFTB/Solver.py:762-772, and eigh at
 // Solver.py:484).  Only the lowest roots are used, so the engine computes the
 // lowest nev eigenpairs on the GPU:
-//   1. Householder reduction to tridiagonal form (one workgroup; the matrix
-//      stays L2-resident, the Householder vector and the product vector in LDS),
+//   1. Householder reduction to tridiagonal form,
 //   2. Sturm-sequence multisection of the wanted eigenvalues (several points per
 //      eigenvalue and round),
 //   3. inverse iteration with partial-pivot tridiagonal LU, vectors of close
@@ -16,8 +15,9 @@
 // eigenpairs of Mh, Rb = Mmsq Tb / sqrt(w), Lb = Mp Rb / w.  The Davidson
 // iterations take the same roots, Rb and Lb from a blocked Cholesky factor of Mm
 // (dftb_subspace_nonhermitian_rl) and Tb once at the end (dftb_subspace_tb).
-// For l >= EIG_MULTI_L the tridiagonalisation runs over many workgroups, one
-// launch per column; the multisection and inverse iteration stay in one.
+// For l >= EIG_MULTI_L the tridiagonalisation runs over many workgroups, one launch per
+// column, until the trailing block fits the LDS of one; the multisection and inverse
+// iteration stay in one.
 #include <math.h>
 #include "common.h"
 #include "gemm.h"
@@ -36,7 +36,8 @@ __global__ __launch_bounds__(EIG_THREADS) void syevx_kernel(const double* __rest
   __shared__ double sp[EIG_MAXL];
   __shared__ double sh[EIG_THREADS / 64];
   __shared__ double s_bnd[2];
-  syevx_block(A, l, ld, nev, evals, evecs, ws, info, sv, sp, sh, s_bnd, EIG_MAXL);
+  __shared__ double stg[EIG_STAGE_WAVES * EIG_STAGE];
+  syevx_block(A, l, ld, nev, evals, evecs, ws, info, sv, sp, sh, s_bnd, EIG_MAXL, stg);
 }
 
 // ---- multi-workgroup Householder reduction (large l) -----------------------
@@ -51,10 +52,10 @@ __global__ __launch_bounds__(EIG_THREADS) void syevx_kernel(const double* __rest
 // Nothing reads what the launch writes: column / row j + 1 are never written
 // (their updated values travel in col), p and col alternate between two buffers,
 // and column j below the subdiagonal receives v_j (rows >= 1) for the
-// back-transformation.  The update term (v_r w_c) + (w_r v_c) is evaluated
-// without contraction, so entries (r, c) and (c, r) stay bitwise equal and row
-// j + 1 is column j + 1 exactly.
+// back-transformation.  Entries (r, c) and (c, r) agree to rounding (the update term's two
+// products are rounded differently), so row j + 1 is column j + 1 to rounding.
 #define HH_THREADS 512
+#define HH_PRE 10   // row entries per lane loaded ahead (rows up to 640)
 
 __global__ __launch_bounds__(256) void sym_copy_kernel(const double* __restrict__ A, int l, int ld, double* __restrict__ W) {
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < (long)l * l; i += (long)gridDim.x * blockDim.x) {
@@ -90,9 +91,10 @@ __device__ double hh_vec(const double* x, int n2, double* sv, double* sh, double
   return 2.0 / vtv;
 }
 
-// (a b) + (c d) rounded without contraction: symmetric in swapping the pairs
+// (a b) + (c d) with the second product rounded, the form every launch of the reduction
+// uses (written out, so that it does not depend on the compiler's choice of contraction)
 __device__ __forceinline__ double sym_upd(double a, double b, double c, double d) {
-  return __dadd_rn(__dmul_rn(a, b), __dmul_rn(c, d));
+  return __builtin_fma(a, b, c * d);
 }
 
 // Step 0's inputs: col = row 0 of W (= column 0), P[r] = t0 (A22 v0)_r.
@@ -124,6 +126,21 @@ __device__ void hh_step_body(double* __restrict__ W, int l, int j, const double*
                              double* __restrict__ hv0, int bid, int nblk, double* sv, double* sw, double* sn,
                              double* sh) {
   const int n2 = l - j - 1, tid = threadIdx.x;
+  const int lane = tid & 63, nw = blockDim.x >> 6;
+  // everything the launch reads is requested before its first reduction: p, the updated
+  // column's row, and the wave's first row (what another XCD wrote comes from memory)
+  const double* rowp = W + (long)(j + 1) * l + (j + 1);
+  const int r0 = 1 + bid * nw + (tid >> 6);
+  double* row0 = W + (long)(j + 1 + r0) * l + (j + 1);
+  double pre[HH_PRE];
+  if (r0 < n2) {
+#pragma unroll
+    for (int q = 0; q < HH_PRE; ++q) {
+      const int c = 1 + lane + 64 * q;
+      if (c < n2) pre[q] = row0[c];
+    }
+  }
+  const double p0 = tid < n2 ? P[tid] : 0.0, rp0 = tid < n2 ? rowp[tid] : 0.0;
   double beta;
   const double t = hh_vec(col + 1, n2, sv, sh, &beta);
   if (bid == 0 && tid == 0) {
@@ -142,7 +159,7 @@ __device__ void hh_step_body(double* __restrict__ W, int l, int j, const double*
   } else {
     double part = 0.0;
     for (int r = tid; r < n2; r += blockDim.x) {
-      const double pr = P[r];
+      const double pr = r == tid ? p0 : P[r];
       sw[r] = pr;
       part += pr * sv[r];
     }
@@ -151,11 +168,10 @@ __device__ void hh_step_body(double* __restrict__ W, int l, int j, const double*
   }
   __syncthreads();
   // updated column j + 1 = updated row j + 1 (rows j + 1 ..)
-  const double* rowp = W + (long)(j + 1) * l + (j + 1);
   const double v0 = sv[0], w0 = sw[0];
   double part = 0.0;
   for (int r = tid; r < n2; r += blockDim.x) {
-    const double a = rowp[r] - sym_upd(v0, sw[r], w0, sv[r]);
+    const double a = (r == tid ? rp0 : rowp[r]) - sym_upd(v0, sw[r], w0, sv[r]);
     if (bid == 0) coln[r] = a;
     if (r >= 1) {
       sn[r - 1] = a;
@@ -174,12 +190,23 @@ __device__ void hh_step_body(double* __restrict__ W, int l, int j, const double*
     if (tid == 0) sn[0] = vn0;
   }
   __syncthreads();
-  const int lane = tid & 63, nw = blockDim.x >> 6;
-  for (int r = 1 + bid * nw + (tid >> 6); r < n2; r += nblk * nw) {
+  for (int r = r0; r < n2; r += nblk * nw) {
     double* row = W + (long)(j + 1 + r) * l + (j + 1);
     const double vr = sv[r], wr = sw[r];
     double s = 0.0;
-    for (int c = 1 + lane; c < n2; c += 64) {
+    int c = 1 + lane;
+    if (r == r0) {
+#pragma unroll
+      for (int q = 0; q < HH_PRE; ++q) {
+        if (c < n2) {
+          const double a = pre[q] - sym_upd(vr, sw[c], wr, sv[c]);
+          row[c] = a;
+          s += a * sn[c - 1];
+        }
+        c += 64;
+      }
+    }
+    for (; c < n2; c += 64) {
       const double a = row[c] - sym_upd(vr, sw[c], wr, sv[c]);
       row[c] = a;
       s += a * sn[c - 1];
@@ -204,11 +231,137 @@ __global__ __launch_bounds__(HH_THREADS) void hh_step_kernel(double* __restrict_
   hh_step_body(W, l, j, col, coln, P, Pn, d, e, tau, hv0, blockIdx.x, gridDim.x, sv, sw, sn, sh);
 }
 
-// The last 2 x 2 block: the updated (l-2, l-2) and (l-1, l-2) from col.
-__global__ void hh_tail_kernel(double* __restrict__ W, int l, const double* __restrict__ col) {
-  if (threadIdx.x == 0) {
-    W[(long)(l - 2) * l + (l - 2)] = col[0];
-    W[(long)(l - 1) * l + (l - 2)] = col[1];
+// Steps j0 .. l - 3 of hh_step in one workgroup with the trailing block in LDS (n0 = l - j0
+// <= HH_LDS_N rows; same operations in the same order, so the results are those of the
+// launches it replaces).  A launch per column costs 5.6 us at any size below ~200; here a
+// column of the last 136 takes 3.6 us.  On entry col / P are step j0's, as for hh_step;
+// the updated last 2 x 2 block goes
+// back to W.
+#define HH_LDS_N 136
+#define HH_LDS_THREADS 1024
+__global__ __launch_bounds__(HH_LDS_THREADS) void hh_finish_kernel(double* __restrict__ W, int l, int j0,
+                                                                   const double* __restrict__ col,
+                                                                   const double* __restrict__ P, double* __restrict__ d,
+                                                                   double* __restrict__ e, double* __restrict__ tau,
+                                                                   double* __restrict__ hv0) {
+  __shared__ double A[HH_LDS_N * HH_LDS_N];   // A[r][c] = W[j0 + 1 + r][j0 + 1 + c]
+  __shared__ double sc[HH_LDS_N + 1], spv[HH_LDS_N], sv[HH_LDS_N], sw[HH_LDS_N], sn[HH_LDS_N];
+  __shared__ double sh[HH_LDS_THREADS / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nw = HH_LDS_THREADS / 64;
+  const int n0 = l - j0 - 1;                  // rows of the trailing block
+  for (int i = tid; i < n0 * n0; i += HH_LDS_THREADS)
+    A[i] = W[(long)(j0 + 1 + i / n0) * l + (j0 + 1 + i % n0)];
+  if (tid <= n0) sc[tid] = col[tid];
+  if (tid < n0) spv[tid] = P[tid];
+  // the sum of one value per thread tid < n2 (blk_sum's order; the other waves add zeros)
+  auto sum = [&](double v, int n2) {
+    __syncthreads();
+    if (wv * 64 < n2) {
+      v = wave_sum(v);
+      if (lane == 0) sh[wv] = v;
+    }
+    __syncthreads();
+    double s = 0.0;
+    for (int i = 0; i * 64 < n2; ++i) s += sh[i];
+    return s;
+  };
+  __syncthreads();
+  for (int j = j0; j + 2 < l; ++j) {
+    const int n2 = l - j - 1, o = j - j0;     // the block's row r is A's row o + r
+    const bool in = tid < n2;
+    const double x = in ? sc[1 + tid] : 0.0, x0 = sc[1], c0 = sc[0], pr = in ? spv[tid] : 0.0;
+    const double al2 = sum(x * x, n2);
+    double t = 0.0, beta = 0.0, v = x;
+    if (al2 > 1e-300) {
+      const double alpha = sqrt(al2);
+      beta = (x0 >= 0.0) ? -alpha : alpha;
+      const double v0 = x0 - beta;
+      t = 2.0 / (al2 - x0 * x0 + v0 * v0);
+      if (tid == 0) v = v0;
+    }
+    if (tid == 0) {
+      tau[j] = t;
+      e[j] = beta;
+      d[j] = c0;
+      hv0[j] = (t == 0.0) ? 0.0 : v;
+    }
+    double w = 0.0;
+    if (t == 0.0) {
+      v = 0.0;                                // nothing to annihilate
+    } else {
+      w = pr;
+      const double K = 0.5 * t * sum(pr * v, n2);
+      w -= K * v;
+    }
+    if (in) {
+      sv[tid] = v;
+      sw[tid] = w;
+    }
+    __syncthreads();
+    const double f0 = sv[0], g0 = sw[0];
+    double a1 = 0.0;
+    if (in) {
+      a1 = A[o * n0 + o + tid] - sym_upd(f0, w, g0, v);
+      sc[tid] = a1;
+      if (tid >= 1) sn[tid - 1] = a1;
+    }
+    const double alpha2 = sum(tid >= 1 ? a1 * a1 : 0.0, n2);
+    const double y0 = sn[0];
+    double tn = 0.0, vn0 = y0;
+    if (alpha2 > 1e-300) {
+      const double alpha = sqrt(alpha2);
+      const double bn = (y0 >= 0.0) ? -alpha : alpha;
+      vn0 = y0 - bn;
+      tn = 2.0 / (alpha2 - y0 * y0 + vn0 * vn0);
+    }
+    // this lane's columns 1 + lane + 64 q of every row
+    constexpr int NQ = (HH_LDS_N + 62) / 64;
+    double cw[NQ], cv[NQ], cn[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const int c = 1 + lane + 64 * q;
+      const bool ok = c < n2;
+      cw[q] = ok ? sw[c] : 0.0;
+      cv[q] = ok ? sv[c] : 0.0;
+      cn[q] = ok ? (c == 1 ? vn0 : sn[c - 1]) : 0.0;
+    }
+    for (int r = 1 + wv; r < n2; r += 2 * nw) {
+      // two rows at a time: their reductions overlap
+      const int r2 = r + nw;
+      const bool two = r2 < n2;
+      double* row = A + (o + r) * n0 + o;
+      double* rowb = A + (o + (two ? r2 : r)) * n0 + o;
+      const double vr = sv[r], wr = sw[r], vb = sv[two ? r2 : r], wb = sw[two ? r2 : r];
+      double s = 0.0, sb = 0.0;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        const int c = 1 + lane + 64 * q;
+        if (c < n2) {
+          const double a = row[c] - sym_upd(vr, cw[q], wr, cv[q]);
+          const double ab = rowb[c] - sym_upd(vb, cw[q], wb, cv[q]);
+          row[c] = a;
+          if (two) rowb[c] = ab;
+          s += a * cn[q];
+          sb += ab * cn[q];
+        }
+      }
+      s = wave_sum(s);
+      sb = wave_sum(sb);
+      if (lane == 0) {
+        spv[r - 1] = tn * s;
+        W[(long)(j + 1 + r) * l + j] = vr;
+        if (two) {
+          spv[r2 - 1] = tn * sb;
+          W[(long)(j + 1 + r2) * l + j] = vb;
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (tid == 0) {
+    W[(long)(l - 2) * l + (l - 2)] = sc[0];
+    W[(long)(l - 1) * l + (l - 2)] = sc[1];
+    W[(long)(l - 1) * l + (l - 1)] = A[n0 * n0 - 1];
   }
 }
 
@@ -237,7 +390,8 @@ __global__ __launch_bounds__(EIG_THREADS) void syevx_vectors_kernel(int l, int n
   __shared__ double sp[EIG_MAXL];
   __shared__ double sh[EIG_THREADS / 64];
   __shared__ double s_bnd[2];
-  syevx_tridiag_vectors(l, nev, evals, ws, sv, sp, sh, s_bnd, EIG_MAXL);
+  __shared__ double stg[EIG_STAGE_WAVES * EIG_STAGE];
+  syevx_tridiag_vectors(l, nev, evals, ws, sv, sp, sh, s_bnd, EIG_MAXL, stg);
 }
 
 __global__ __launch_bounds__(EIG_THREADS) void syevx_back_kernel(int l, int nev, double* __restrict__ evecs,
@@ -330,14 +484,16 @@ extern "C" int dftb_syevx(const double* A, int l, int ld, int nev, double* evals
     if (g > 256) g = 256;
     hipLaunchKernelGGL(hh_start_kernel, dim3(g), dim3(HH_THREADS), 0, st, (const double*)W, l, C2[0], P2[0]);
   }
-  for (int j = 0; j + 2 < l; ++j) {
+  const int j0 = l - 1 > HH_LDS_N ? l - 1 - HH_LDS_N : 0;
+  for (int j = 0; j < j0; ++j) {
     const int rows = l - j - 2;             // rows updated (the first row of the block is not)
     int g = (rows + waves - 1) / waves;
     if (g > 256) g = 256;
     hipLaunchKernelGGL(hh_step_kernel, dim3(g), dim3(HH_THREADS), 0, st, W, l, j, (const double*)C2[j & 1],
                        C2[(j + 1) & 1], (const double*)P2[j & 1], P2[(j + 1) & 1], d, e, tau, hv0);
   }
-  hipLaunchKernelGGL(hh_tail_kernel, dim3(1), dim3(64), 0, st, W, l, (const double*)C2[(l - 2) & 1]);
+  hipLaunchKernelGGL(hh_finish_kernel, dim3(1), dim3(HH_LDS_THREADS), 0, st, W, l, j0, (const double*)C2[j0 & 1],
+                     (const double*)P2[j0 & 1], d, e, tau, hv0);
   hipLaunchKernelGGL(hh_rows_kernel, dim3(ceil_div((long)l * l, 256) < 4096 ? ceil_div((long)l * l, 256) : 4096),
                      dim3(256), 0, st, W, l, (const double*)hv0);
   hipLaunchKernelGGL(syevx_vectors_kernel, dim3(1), dim3(EIG_THREADS), 0, st, l, nev, evals, ws);
@@ -674,13 +830,24 @@ __global__ void fill_zero_kernel(double* X, long n) {
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) X[i] = 0.0;
 }
 
+// the value of `lane` in every lane, through scalar registers
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
 // Factor the b x b diagonal block at (p, p) of W (lower triangle, trailing updates
-// applied) into L[p.., p..] (zeros above the diagonal).  One wave: lane i holds row
-// i in registers and column k travels by lane shuffles.  A non-positive pivot sets
-// info (DFTB_ERR_NOT_SPD, pivot index) and continues with a unit pivot, so that
-// later launches see finite values.
+// applied) into L[p.., p..] (zeros above the diagonal) and, with Linv, its inverse
+// (b x b, zeros above the diagonal).  One wave: lane i holds row i in registers, and an
+// entry needed by all lanes travels through scalar registers (v_readlane; with
+// ds_bpermute shuffles for the factor and LDS reads for the inverse the two took 87 and 52
+// us per block, as two launches; now 54 us together).  The inverse is column-oriented
+// forward substitution, lane c forming column c.  Entries above the diagonal are carried
+// along unused.  A non-positive pivot sets info (DFTB_ERR_NOT_SPD, pivot index) and
+// continues with a unit pivot, so that later launches see finite values.
 __global__ __launch_bounds__(64) void chol_diag_kernel(const double* __restrict__ W, double* __restrict__ L, int l,
-                                                       int p, int b, int* __restrict__ info) {
+                                                       int p, int b, double* __restrict__ Linv,
+                                                       int* __restrict__ info) {
   const int i = threadIdx.x;
   double row[CHOL_NB];
 #pragma unroll
@@ -689,7 +856,7 @@ __global__ __launch_bounds__(64) void chol_diag_kernel(const double* __restrict_
 #pragma unroll
   for (int k = 0; k < CHOL_NB; ++k) {
     if (k < b) {
-      double d = __shfl(row[k], k, 64);
+      double d = lane_value(row[k], k);
       if (!(d > 0.0)) {
         if (bad < 0) bad = k;
         d = 1.0;
@@ -698,10 +865,7 @@ __global__ __launch_bounds__(64) void chol_diag_kernel(const double* __restrict_
       const double lik = (i == k) ? piv : (i > k ? row[k] / piv : 0.0);
       row[k] = lik;
 #pragma unroll
-      for (int j = k + 1; j < CHOL_NB; ++j) {
-        const double ljk = __shfl(lik, j, 64);
-        if (i >= j) row[j] -= lik * ljk;
-      }
+      for (int j = k + 1; j < CHOL_NB; ++j) row[j] -= lik * lane_value(lik, j);
     }
   }
   if (i == 0 && bad >= 0 && info[0] == 0) {
@@ -712,27 +876,17 @@ __global__ __launch_bounds__(64) void chol_diag_kernel(const double* __restrict_
 #pragma unroll
     for (int j = 0; j < CHOL_NB; ++j)
       if (j < b) L[(long)(p + i) * l + (p + j)] = (j <= i) ? row[j] : 0.0;
-}
-
-// Linv (b x b) = inverse of the factor block L[p.., p..]: one wave, lane c forms
-// column c by column-oriented forward substitution (rows of the factor read from
-// LDS at uniform addresses); entries above the diagonal come out zero.
-__global__ __launch_bounds__(64) void chol_inv_kernel(const double* __restrict__ L, int l, int p, int b,
-                                                      double* __restrict__ Linv) {
-  __shared__ double sL[CHOL_NB][CHOL_NB + 1];
-  const int i = threadIdx.x;
-  for (int j = 0; j < CHOL_NB; ++j) sL[i][j] = (i < b && j < b) ? L[(long)(p + i) * l + (p + j)] : 0.0;
-  __syncthreads();
+  if (!Linv) return;
   double x[CHOL_NB];
 #pragma unroll
   for (int r = 0; r < CHOL_NB; ++r) x[r] = (r == i) ? 1.0 : 0.0;
 #pragma unroll
   for (int k = 0; k < CHOL_NB; ++k) {
     if (k < b) {
-      const double xk = x[k] / sL[k][k];
+      const double xk = x[k] / lane_value(row[k], k);
       x[k] = xk;
 #pragma unroll
-      for (int r = k + 1; r < CHOL_NB; ++r) x[r] -= sL[r][k] * xk;
+      for (int r = k + 1; r < CHOL_NB; ++r) x[r] -= lane_value(row[k], r) * xk;
     }
   }
   if (i < b)
@@ -751,12 +905,11 @@ static int cholesky_blocked(const double* Mm, int l, int ld, double* W, double* 
   int rc;
   for (int p = 0; p < l; p += CHOL_NB) {
     const int b = l - p < CHOL_NB ? l - p : CHOL_NB;
-    hipLaunchKernelGGL(chol_diag_kernel, dim3(1), dim3(64), 0, st, (const double*)W, L, l, p, b, info);
-    DFTB_CHECK_LAUNCH();
     const int r = l - p - b;
-    if (r <= 0) break;
-    hipLaunchKernelGGL(chol_inv_kernel, dim3(1), dim3(64), 0, st, (const double*)L, l, p, b, Linv);
+    hipLaunchKernelGGL(chol_diag_kernel, dim3(1), dim3(64), 0, st, (const double*)W, L, l, p, b,
+                       r > 0 ? Linv : (double*)nullptr, info);
     DFTB_CHECK_LAUNCH();
+    if (r <= 0) break;
     // panel: L21 = W21 L11^{-T}
     GemmArgs g = gemm_args_default();
     g.A = W + (long)(p + b) * l + p; g.lda = l;

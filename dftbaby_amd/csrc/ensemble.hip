@@ -350,7 +350,7 @@ __device__ int ens_orthonormalize(const double* B, int l, double* Q, int m, long
 // --------------------------------------------------------------------------
 template <typename T>
 __device__ void ens_davidson(const EnsMolecule& Mo, double conv, int maxiter, double* sh, double* sv, double* sp,
-                             double* bnd, int* s_sel) {
+                             double* bnd, int* s_sel, double* stg) {
   char* ws = (char*)Mo.work;
   const EnsLayout L = ens_layout(Mo);
   const long N = (long)Mo.opad * Mo.vpad;
@@ -430,7 +430,7 @@ __device__ void ens_davidson(const EnsMolecule& Mo, double conv, int maxiter, do
       break;
     }
     const int nev = k < l ? k : l;
-    syevx_block(H, l, l, nev, w2, Tb, ws + L.eig, nullptr, sv, sp, sh, bnd, ENS_MAXL);
+    syevx_block(H, l, l, nev, w2, Tb, ws + L.eig, nullptr, sv, sp, sh, bnd, ENS_MAXL, stg);
     __syncthreads();
     int bad = 0;
     for (int n = threadIdx.x; n < nev; n += blockDim.x)
@@ -556,13 +556,14 @@ __global__ __launch_bounds__(ENS_THREADS) void ensemble_kernel(const EnsMolecule
   __shared__ double sp[ENS_MAXL];
   __shared__ double bnd[2];
   __shared__ int s_sel[1 + 2 * ENS_MAXK];
+  __shared__ double stg[EIG_STAGE_WAVES * EIG_STAGE];
   const int mi = blockIdx.x;
   if (mi >= nmol) return;
   const EnsMolecule& Mo = mols[mi];
   if (Mo.precision == 1)
-    ens_davidson<float>(Mo, conv, maxiter, sh, sv, sp, bnd, s_sel);
+    ens_davidson<float>(Mo, conv, maxiter, sh, sv, sp, bnd, s_sel, stg);
   else
-    ens_davidson<double>(Mo, conv, maxiter, sh, sv, sp, bnd, s_sel);
+    ens_davidson<double>(Mo, conv, maxiter, sh, sv, sp, bnd, s_sel, stg);
 }
 
 extern "C" int dftb_ensemble_solve(const EnsMolecule* mols_dev, int nmol, double conv, int maxiter, void* stream) {
