@@ -18,78 +18,229 @@
 #define ENS_MAXK 32     // largest number of states
 
 // --------------------------------------------------------------------------
-// block-level MFMA GEMM with direct (L2/L1-cached) operand loads
+// block-level MFMA GEMM on global operands
 //   C = alpha op(A) op(B) + beta C; optional column remap of the output:
 //   col -> (col / cdiv) * cstr + row * ldc + col % cdiv.
+// The eight waves deal out tiles of TM x TN 16 x 16 blocks; a wave loads its operand
+// fragments straight into registers, KS chunks of 16 k ahead of the MFMAs (two buffers).
+// Every result is one chain over ascending k (an MFMA adds its four k in lane-group order),
+// so the tile shape does not show in the results.  One CU sustains 614 GFLOP/s in FP32 and
+// 307 in FP64; latency of the loads bounds these products.  With 32 x 32 tiles loaded and
+// multiplied in turn the block products of a C22H24 member (FP32 exchange, 17 iterations) took
+// 188 ms and its Newton-Schulz products 91 ms; with these tiles 127 and 82 ms.
 // --------------------------------------------------------------------------
-template <typename T>
-__device__ __forceinline__ T ld_op(const T* X, long ld, int trans, long r, long c) {
-  return trans ? X[c * ld + r] : X[r * ld + c];
+typedef double ens_d2 __attribute__((ext_vector_type(2), aligned(8)));
+typedef float ens_f2 __attribute__((ext_vector_type(2), aligned(4)));
+template <typename T> struct EnsVec;
+template <> struct EnsVec<double> { typedef ens_d2 pair; typedef d4_t acc; };
+template <> struct EnsVec<float> { typedef ens_f2 pair; typedef f4_t acc; };
+
+__device__ __forceinline__ void ens_swap16(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap((unsigned)__float_as_uint(a), (unsigned)__float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void ens_swap16(double& a, double& b) {
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(a), (unsigned)__double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(a), (unsigned)__double2hiint(b), false, false);
+  a = __hiloint2double((int)hi[0], (int)lo[0]);
+  b = __hiloint2double((int)hi[1], (int)lo[1]);
+}
+__device__ __forceinline__ d4_t ens_mfma(double a, double b, d4_t c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f4_t ens_mfma(float a, float b, f4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// N 16-row fragments of one operand over KS chunks.  KC: K contiguous (x[row * ld + k]), loaded as
+// pairs that one lane swap brings to k = 16 c + 4 s + lane / 16; otherwise x[k * ld + row].
+// Rows beyond the operand repeat the last one (their results are not stored).
+template <typename T, int N, int KS, bool KC>
+struct EnsFrag {
+  const T* ptr[N];
+  long ld;
+  __device__ __forceinline__ void init(const T* x, long ld_, int r0, int rows, int lane) {
+    ld = ld_;
+    const int g = lane >> 4, k = KC ? 2 * (((g & 1) << 1) | (g >> 1)) : g;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      int r = r0 + 16 * i + (lane & 15);
+      if (r >= rows) r = rows - 1;
+      ptr[i] = KC ? x + r * ld + k : x + k * ld + r;
+    }
+  }
+  __device__ __forceinline__ void load(long k0, T (&v)[N][4 * KS]) const {
+#pragma unroll
+    for (int h = 0; h < 2 * KS; ++h)
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        if constexpr (KC) {
+          const auto x = *(const typename EnsVec<T>::pair*)(ptr[i] + k0 + 8 * h);
+          v[i][2 * h] = x.x;
+          v[i][2 * h + 1] = x.y;
+        } else {
+          const T* q = ptr[i] + (k0 + 8 * h) * ld;
+          v[i][2 * h] = q[0];
+          v[i][2 * h + 1] = q[4 * ld];
+        }
+      }
+  }
+  __device__ __forceinline__ void order(T (&v)[N][4 * KS]) const {
+    if constexpr (KC) {
+#pragma unroll
+      for (int h = 0; h < 2 * KS; ++h)
+#pragma unroll
+        for (int i = 0; i < N; ++i) ens_swap16(v[i][2 * h], v[i][2 * h + 1]);
+    }
+  }
+  // one chunk at k0 with zeros from kend on, in MFMA order
+  __device__ __forceinline__ void load_chunk(int k0, int kend, int lane, T (&v)[N][4 * KS]) const {
+    const int g = lane >> 4, kp = KC ? 2 * (((g & 1) << 1) | (g >> 1)) : g;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int k = k0 + 4 * s + g;
+        v[i][s] = k < kend ? (KC ? ptr[i][k - kp] : ptr[i][(k - kp) * ld]) : (T)0;
+      }
+  }
+};
+
+template <typename T, typename TC, int TM, int TN, int KS, bool AT, bool BT>
+__device__ __forceinline__ void bgemm_tiles(int M, int N, int K, const T* __restrict__ A, long lda,
+                                            const T* __restrict__ B, long ldb, TC* __restrict__ C, long ldc,
+                                            double alpha, double beta, long cdiv, long cstr) {
+  const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int tm = (M + 16 * TM - 1) / (16 * TM), tn = (N + 16 * TN - 1) / (16 * TN);
+  constexpr bool F64 = sizeof(T) == 8;
+  const int ns = K / (16 * KS);
+  for (int t = wv; t < tm * tn; t += nw) {
+    const int m0 = (t / tn) * 16 * TM, n0 = (t % tn) * 16 * TN;
+    EnsFrag<T, TM, KS, !AT> fa;
+    EnsFrag<T, TN, KS, BT> fb;
+    fa.init(A, lda, m0, M, lane);
+    fb.init(B, ldb, n0, N, lane);
+    typename EnsVec<T>::acc acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = (typename EnsVec<T>::acc)((T)0);
+    auto mul = [&](T (&a)[TM][4 * KS], T (&b)[TN][4 * KS], int steps) {
+#pragma unroll
+      for (int s = 0; s < 4 * KS; ++s)
+        if (s < steps)
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = ens_mfma(a[i][s], b[j][s], acc[i][j]);
+    };
+    T av[TM][4 * KS], bv[TN][4 * KS];
+    if (ns > 0) {
+      // two buffers; the odd one goes first, and the last prefetch repeats the last chunks
+      T aw[TM][4 * KS], bw[TN][4 * KS];
+      long k = 0;
+      fa.load(k, av);
+      fb.load(k, bv);
+      if (ns & 1) {
+        fa.order(av);
+        fb.order(bv);
+        mul(av, bv, 4 * KS);
+        if (ns > 1) k += 16 * KS;
+        fa.load(k, av);
+        fb.load(k, bv);
+      }
+      for (int c = ns & 1; c < ns; c += 2) {
+        k += 16 * KS;
+        fa.load(k, aw);
+        fb.load(k, bw);
+        __builtin_amdgcn_sched_barrier(0);
+        fa.order(av);
+        fb.order(bv);
+        mul(av, bv, 4 * KS);
+        __builtin_amdgcn_sched_barrier(0);
+        if (c + 2 < ns) k += 16 * KS;
+        fa.load(k, av);
+        fb.load(k, bv);
+        __builtin_amdgcn_sched_barrier(0);
+        fa.order(aw);
+        fb.order(bw);
+        mul(aw, bw, 4 * KS);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    for (int k = ns * 16 * KS; k < K; k += 16) {
+      fa.load_chunk(k, K, lane, av);
+      fb.load_chunk(k, K, lane, bv);
+      mul(av, bv, 4);
+    }
+    long coff[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int col = n0 + 16 * j + (lane & 15);
+      coff[j] = cdiv > 0 ? (col / (int)cdiv) * cstr + col % (int)cdiv : col;
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        // v_mfma_f64_16x16x4f64 holds rows (lane/16) + 4r, the f32 form rows 4(lane/16) + r
+        const int row = m0 + 16 * i + (F64 ? ((lane >> 4) + 4 * r) : (4 * (lane >> 4) + r));
+        if (row < M)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            if (n0 + 16 * j + (lane & 15) < N) {
+              const long off = row * ldc + coff[j];
+              double v = alpha * (double)acc[i][j][r];
+              if (beta != 0.0) v += beta * (double)C[off];
+              C[off] = (TC)v;
+            }
+      }
+  }
+}
+
+// cycles of the product over the eight waves (two per SIMD) with TM x TN tiles: MFMA time of
+// a SIMD, operands at about 40 bytes per cycle and CU, or memory latency per buffer
+__device__ __forceinline__ float bgemm_cost(int M, int N, int K, int tm, int tn, int ks, int esz) {
+  const int nt = ((M + 16 * tm - 1) / (16 * tm)) * ((N + 16 * tn - 1) / (16 * tn));
+  const int act = nt < 8 ? nt : 8;
+  const float mf = (esz == 8 ? 256.0f : 128.0f) * tm * tn, op = act * (tm + tn) * 256.0f * esz / 40.0f;
+  float w = (act > 4 ? 2.0f : 1.0f) * mf;
+  w = fmaxf(w, fmaxf(op, mf + 500.0f / ks));
+  return ((nt + 7) / 8) * (((K + 15) / 16) * w + 1500.0f + 60.0f * tm * tn);
+}
+
+template <typename T, typename TC, bool AT, bool BT>
+__device__ __noinline__ void bgemm_t(int M, int N, int K, const T* __restrict__ A, long lda, const T* __restrict__ B,
+                                     long ldb, TC* __restrict__ C, long ldc, double alpha, double beta, long cdiv,
+                                     long cstr) {
+  constexpr int E = sizeof(T);
+  constexpr int KB = E == 8 ? 2 : 4;          // chunks per buffer of the 32 x 32 tile
+  const float c11 = bgemm_cost(M, N, K, 1, 1, 4, E), c12 = bgemm_cost(M, N, K, 1, 2, KB, E);
+  const float c22 = bgemm_cost(M, N, K, 2, 2, KB, E), c24 = bgemm_cost(M, N, K, 2, 4, KB / 2, E);
+  const float best = fminf(fminf(c11, c12), fminf(c22, c24));
+  if (best == c24)
+    bgemm_tiles<T, TC, 2, 4, KB / 2, AT, BT>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr);
+  else if (best == c22)
+    bgemm_tiles<T, TC, 2, 2, KB, AT, BT>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr);
+  else if (best == c12)
+    bgemm_tiles<T, TC, 1, 2, KB, AT, BT>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr);
+  else
+    bgemm_tiles<T, TC, 1, 1, 4, AT, BT>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr);
+  __syncthreads();
 }
 
 template <typename T, typename TC>
-__device__ __noinline__ void bgemm(int M, int N, int K, const T* __restrict__ A, long lda, int at,
-                                   const T* __restrict__ B, long ldb, int bt, TC* __restrict__ C, long ldc,
-                                   double alpha, double beta, long cdiv, long cstr) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  const int tm = (M + 31) / 32, tn = (N + 31) / 32;
-  constexpr bool F64 = sizeof(T) == 8;
-  for (int t = wv; t < tm * tn; t += nw) {
-    const int m0 = (t / tn) * 32, n0 = (t % tn) * 32;
-    d4_t acc[2][2];
-    f4_t accf[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        acc[i][j] = (d4_t)(0.0);
-        accf[i][j] = (f4_t)(0.0f);
-      }
-    const int mr0 = m0 + (lane & 15), nr0 = n0 + (lane & 15);
-    for (int k0 = 0; k0 < K; k0 += 16) {
-      T a[4][2], b[4][2];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int kk = k0 + 4 * u + (lane >> 4);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int m = mr0 + 16 * i;
-          a[u][i] = (m < M && kk < K) ? ld_op(A, lda, at, m, kk) : (T)0;
-          const int n = nr0 + 16 * i;
-          b[u][i] = (n < N && kk < K) ? ld_op(B, ldb, bt, kk, n) : (T)0;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            if constexpr (F64)
-              acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[u][i], (double)b[u][j], acc[i][j], 0, 0, 0);
-            else
-              accf[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)a[u][i], (float)b[u][j], accf[i][j], 0, 0, 0);
-          }
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          // v_mfma_f64_16x16x4f64 holds rows (lane/16) + 4r, the f32 form rows 4(lane/16) + r
-          const int rr = F64 ? ((lane >> 4) + 4 * r) : (4 * (lane >> 4) + r);
-          const long row = m0 + 16 * i + rr;
-          const long col = n0 + 16 * j + (lane & 15);
-          if (row < M && col < N) {
-            const long off = cdiv > 0 ? (col / cdiv) * cstr + row * ldc + col % cdiv : row * ldc + col;
-            double v = alpha * (F64 ? (double)acc[i][j][r] : (double)accf[i][j][r]);
-            if (beta != 0.0) v += beta * (double)C[off];
-            C[off] = (TC)v;
-          }
-        }
-  }
-  __syncthreads();
+__device__ __forceinline__ void bgemm(int M, int N, int K, const T* A, long lda, int at, const T* B, long ldb, int bt,
+                                      TC* C, long ldc, double alpha, double beta, long cdiv, long cstr) {
+  // the three operand orders in use (constant at every call)
+  if (at)
+    bgemm_t<T, TC, true, false>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr);
+  else if (bt)
+    bgemm_t<T, TC, false, true>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr);
+  else
+    bgemm_t<T, TC, false, false>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr);
 }
 
 template <typename T, typename TC>
@@ -294,12 +445,14 @@ __device__ int ens_orthonormalize(const double* B, int l, double* Q, int m, long
   }
   for (int pass = 0; pass < 2; ++pass) {
     bg<double, double>(m, m, (int)N, Q, N, 0, Q, N, 1, G, m);
-    if (threadIdx.x == 0) {
-      for (int i = 0; i < m * m; ++i) {
-        Lc[i] = 0.0;
-        Li[i] = 0.0;
-      }
-      for (int j = 0; j < m; ++j) {
+    for (int i = threadIdx.x; i < m * m; i += blockDim.x) {
+      Lc[i] = 0.0;
+      Li[i] = 0.0;
+    }
+    __syncthreads();
+    // column by column, one row per thread; then the inverse, one column per thread
+    for (int j = 0; j < m; ++j) {
+      if (threadIdx.x == 0) {
         double d = G[j * m + j];
         for (int q = 0; q < j; ++q) d -= Lc[j * m + q] * Lc[j * m + q];
         const double r = pass == 0 ? ref[j] * ref[j] : 1.0;
@@ -307,26 +460,25 @@ __device__ int ens_orthonormalize(const double* B, int l, double* Q, int m, long
         const int ok = keep[j] && d > t2 * r && d > 1e-12 * G[j * m + j] && d > 0.0;
         keep[j] = ok;
         Lc[j * m + j] = ok ? sqrt(d) : 1.0;
-        for (int i = j + 1; i < m; ++i) {
-          double s = 0.0;
-          if (ok) {
-            s = G[i * m + j];
-            for (int q = 0; q < j; ++q) s -= Lc[i * m + q] * Lc[j * m + q];
-            s /= Lc[j * m + j];
-          }
-          Lc[i * m + j] = s;
-        }
       }
-      for (int c = 0; c < m; ++c)
-        for (int i = c; i < m; ++i) {
-          double s = (i == c) ? 1.0 : 0.0;
-          for (int q = c; q < i; ++q) s -= Lc[i * m + q] * Li[q * m + c];
-          Li[i * m + c] = s / Lc[i * m + i];
+      __syncthreads();
+      if (keep[j])
+        for (int i = j + 1 + threadIdx.x; i < m; i += blockDim.x) {
+          double s = G[i * m + j];
+          for (int q = 0; q < j; ++q) s -= Lc[i * m + q] * Lc[j * m + q];
+          Lc[i * m + j] = s / Lc[j * m + j];
         }
-      for (int i = 0; i < m; ++i)
-        if (!keep[i])
-          for (int c = 0; c < m; ++c) Li[i * m + c] = 0.0;
+      __syncthreads();
     }
+    for (int c = threadIdx.x; c < m; c += blockDim.x)
+      for (int i = c; i < m; ++i) {
+        double s = (i == c) ? 1.0 : 0.0;
+        for (int q = c; q < i; ++q) s -= Lc[i * m + q] * Li[q * m + c];
+        Li[i * m + c] = s / Lc[i * m + i];
+      }
+    __syncthreads();
+    for (int i = threadIdx.x; i < m * m; i += blockDim.x)
+      if (!keep[i / m]) Li[i] = 0.0;
     __syncthreads();
     bg<double, double>(m, (int)N, m, Li, m, 0, Q, N, 0, Qt, N);
     for (long i = threadIdx.x; i < (long)m * N; i += blockDim.x) Q[i] = Qt[i];

@@ -38,3 +38,19 @@ def test_ensemble_reports_nonconvergence():
     ops = build_operators([ground_state("C8H10", 1, 0.05, 1)])
     with pytest.raises(ExcitedStatesNotConverged):
         solve_operators(ops, 4, conv=1e-14, maxiter=1)
+
+
+@pytest.mark.parametrize("copies", [1, 30, 100])
+@pytest.mark.parametrize("precision,conv,tol", [(0, 1e-8, 1e-9), (1, 1e-6, 1e-6)])
+def test_ensemble_batch_size_does_not_show(copies, precision, conv, tol):
+    """A member's results are those of the oracle (energies within the bounds above) and the
+    same bits alone and in a batch of any size."""
+    from dftbaby_amd.ensemble import build_operators, solve_operators
+    for name, n in (("C8H10", copies), ("C12H14", min(copies, 2))):
+        gs = ground_state(name, 1, 0.05, 7)
+        res = solve_operators(build_operators([gs] * n), 5, conv=conv, maxiter=100, precision=precision)
+        ref_w, _ = _oracle(gs, 5, 1e-8)
+        alone = solve_operators(build_operators([gs]), 5, conv=conv, maxiter=100, precision=precision)
+        for w, xpy in zip(res.Omega, res.XpY):
+            assert np.abs(w - ref_w).max() < tol, (w, ref_w)
+            assert np.array_equal(w, alone.Omega[0]) and np.array_equal(xpy, alone.XpY[0])
