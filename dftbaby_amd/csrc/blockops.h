@@ -357,40 +357,24 @@ __device__ void cluster_wave(int l, int nev, int m0, int m1, const double* __res
   }
 }
 
-// Lowest nev eigenpairs of the symmetric l x l matrix A (leading dim ld), one
-// workgroup: Householder tridiagonalisation, Sturm bisection, inverse
-// iteration (clusters re-orthogonalised), back-transformation.  sv, sp: LDS
-// scratch of cap >= l doubles each; sh: >= blockDim/64 doubles; s_bnd: 2; stg:
-// EIG_STAGE_WAVES * EIG_STAGE doubles of LDS.
-__device__ __noinline__ void syevx_tail(int l, int nev, double* __restrict__ evals, double* __restrict__ evecs,
-                                        char* __restrict__ ws, int* __restrict__ info, double* sv, double* sp,
-                                        double* sh, double* s_bnd, int cap, double* stg);
-
-__device__ __noinline__ void syevx_block(const double* __restrict__ A, int l, int ld, int nev,
-                                         double* __restrict__ evals, double* __restrict__ evecs,
-                                         char* __restrict__ ws, int* __restrict__ info, double* sv, double* sp,
-                                         double* sh, double* s_bnd, int cap, double* stg) {
-  EigLayout Lo = eig_layout(l, nev);
-  double* W = (double*)(ws + Lo.W);
-  double* d = (double*)(ws + Lo.d);
-  double* e = (double*)(ws + Lo.e);
-  double* tau = (double*)(ws + Lo.tau);
-  double* Z = (double*)(ws + Lo.z);
-  double* scr = (double*)(ws + Lo.scratch);
+// Householder steps j0 <= j < j1 in one workgroup.  X(r, c) = X[r * ldx + c] holds the rows and
+// columns j0, .. l - 1 of the matrix, in LDS or in global memory; reflector j goes to row j of W
+// behind the diagonal (never read again by the reduction), where the back-transformation reads it
+// coalesced.  A wave takes RB rows and CB chunks of 64 columns at a time: a load's latency, not its
+// bandwidth, bounds a step.
+template <int RB, int CB, typename P>
+__device__ __forceinline__ void hh_block_steps(P X, int ldx, int j0, int j1, int l, double* __restrict__ W,
+                                               double* __restrict__ d, double* __restrict__ e,
+                                               double* __restrict__ tau, lds_f64* sv, lds_f64* sp, double* sh) {
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nw = blockDim.x >> 6;
-
-  for (long i = tid; i < (long)l * l; i += blockDim.x) {
-    long r = i / l, c = i % l;
-    W[i] = 0.5 * (A[r * ld + c] + A[c * ld + r]);
-  }
-  __syncthreads();
-
-  // ---- 1. Householder tridiagonalisation
-  for (int j = 0; j + 2 < l; ++j) {
+  for (int j = j0; j < j1; ++j) {
     const int n2 = l - j - 1;
+    P X2 = X + (j + 1 - j0) * (ldx + 1);       // the trailing block
+    double* refl = W + (long)j * l + j + 1;
+    const double dj = X[(j - j0) * (ldx + 1)];
     double part = 0.0;
     for (int r = tid; r < n2; r += blockDim.x) {
-      double x = W[(long)(j + 1 + r) * l + j];
+      const double x = X2[r * ldx - 1];
       sv[r] = x;
       part += x * x;
     }
@@ -398,8 +382,8 @@ __device__ __noinline__ void syevx_block(const double* __restrict__ A, int l, in
     const double x0 = sv[0];
     __syncthreads();
     if (alpha2 <= 1e-300) {
-      if (tid == 0) { tau[j] = 0.0; e[j] = 0.0; d[j] = W[(long)j * l + j]; }
-      for (int r = tid; r < n2; r += blockDim.x) W[(long)(j + 1 + r) * l + j] = 0.0;
+      if (tid == 0) { tau[j] = 0.0; e[j] = 0.0; d[j] = dj; }
+      for (int r = tid; r < n2; r += blockDim.x) refl[r] = 0.0;
       __syncthreads();
       continue;
     }
@@ -408,30 +392,197 @@ __device__ __noinline__ void syevx_block(const double* __restrict__ A, int l, in
     const double v0 = x0 - beta;
     const double vtv = alpha2 - x0 * x0 + v0 * v0;
     const double t = 2.0 / vtv;
-    if (tid == 0) { sv[0] = v0; tau[j] = t; e[j] = beta; d[j] = W[(long)j * l + j]; }
+    if (tid == 0) { sv[0] = v0; tau[j] = t; e[j] = beta; d[j] = dj; }
     __syncthreads();
-    // p = t * A22 v  (one wave per row, lanes across columns)
-    for (int r = wv; r < n2; r += nw) {
-      const double* row = W + (long)(j + 1 + r) * l + (j + 1);
-      double s = 0.0;
-      for (int c = lane; c < n2; c += 64) s += row[c] * sv[c];
-      s = wave_sum(s);
-      if (lane == 0) sp[r] = t * s;
+    // p = t * A22 v  (lanes across columns)
+    for (int r = RB * wv; r < n2; r += RB * nw) {
+      double s[RB];
+      int o[RB];
+#pragma unroll
+      for (int u = 0; u < RB; ++u) {
+        s[u] = 0.0;
+        o[u] = (r + u < n2 ? r + u : n2 - 1) * ldx;
+      }
+      for (int c0 = lane; c0 < n2; c0 += 64 * CB) {
+        double x[CB][RB];
+#pragma unroll
+        for (int q = 0; q < CB; ++q) {
+          const int c = c0 + 64 * q < n2 ? c0 + 64 * q : c0;
+#pragma unroll
+          for (int u = 0; u < RB; ++u) x[q][u] = X2[o[u] + c];
+        }
+#pragma unroll
+        for (int q = 0; q < CB; ++q)
+          if (c0 + 64 * q < n2) {
+            const double v = sv[c0 + 64 * q];
+#pragma unroll
+            for (int u = 0; u < RB; ++u) s[u] += x[q][u] * v;
+          }
+      }
+#pragma unroll
+      for (int u = 0; u < RB; ++u) s[u] = wave_sum(s[u]);
+      if (lane == 0) {
+#pragma unroll
+        for (int u = 0; u < RB; ++u)
+          if (r + u < n2) sp[r + u] = t * s[u];
+      }
     }
     __syncthreads();
     part = 0.0;
     for (int r = tid; r < n2; r += blockDim.x) part += sp[r] * sv[r];
     const double K = 0.5 * t * blk_sum(part, sh);
-    for (int r = tid; r < n2; r += blockDim.x) sp[r] -= K * sv[r];
-    __syncthreads();
-    for (long i = tid; i < (long)n2 * n2; i += blockDim.x) {
-      int r = (int)(i / n2), c = (int)(i % n2);
-      W[(long)(j + 1 + r) * l + (j + 1 + c)] -= sv[r] * sp[c] + sp[r] * sv[c];
+    for (int r = tid; r < n2; r += blockDim.x) {
+      refl[r] = sv[r];
+      sp[r] -= K * sv[r];
     }
-    for (int r = tid; r < n2; r += blockDim.x) W[(long)(j + 1 + r) * l + j] = sv[r];
+    __syncthreads();
+    for (int r = RB * wv; r < n2; r += RB * nw) {
+      double vr[RB], pr[RB];
+      int o[RB];
+#pragma unroll
+      for (int u = 0; u < RB; ++u) {
+        const int q = r + u < n2 ? r + u : n2 - 1;
+        vr[u] = sv[q];
+        pr[u] = sp[q];
+        o[u] = q * ldx;
+      }
+      for (int c0 = lane; c0 < n2; c0 += 64 * CB) {
+        double x[CB][RB];
+#pragma unroll
+        for (int q = 0; q < CB; ++q) {
+          const int c = c0 + 64 * q < n2 ? c0 + 64 * q : c0;
+#pragma unroll
+          for (int u = 0; u < RB; ++u) x[q][u] = X2[o[u] + c];
+        }
+#pragma unroll
+        for (int q = 0; q < CB; ++q)
+          if (c0 + 64 * q < n2) {
+            const double vc = sv[c0 + 64 * q], pc = sp[c0 + 64 * q];
+#pragma unroll
+            for (int u = 0; u < RB; ++u)   // rows beyond the last repeat it: the same value again
+              X2[o[u] + c0 + 64 * q] = x[q][u] - __builtin_fma(vr[u], pc, pr[u] * vc);
+          }
+      }
+    }
     __syncthreads();
   }
-  syevx_tail(l, nev, evals, evecs, ws, info, sv, sp, sh, s_bnd, cap, stg);
+}
+
+// z <- H_0 ... H_{l-3} z, one wave per vector: entry i of vector n at Z[i * zi + n * zn], reflectors
+// in the rows of W behind the diagonal, the next one's first 256 entries loaded ahead.
+template <typename P>
+__device__ __forceinline__ void hh_block_back(int l, int nev, const double* __restrict__ W,
+                                              const double* __restrict__ tau, P Z, int zi, int zn) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  for (int n = wv; n < nev; n += nw) {
+    P z = Z + n * zn;
+    double vn[4], tn = 0.0;
+    auto fetch = [&](int j) {
+      tn = tau[j];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int i = j + 1 + lane + 64 * q;
+        vn[q] = i < l ? W[(long)j * l + i] : 0.0;
+      }
+    };
+    if (l >= 3) fetch(l - 3);
+    for (int j = l - 3; j >= 0; --j) {
+      const int n2 = l - j - 1;
+      const double t = tn;
+      double v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] = vn[q];
+      if (j > 0) fetch(j - 1);
+      if (t == 0.0) continue;
+      const double* vr = W + (long)j * l + j + 1;
+      P zj = z + (j + 1) * zi;
+      double s = 0.0, x[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int r = lane + 64 * q;
+        x[q] = r < n2 ? zj[r * zi] : 0.0;
+        if (r < n2) s += v[q] * x[q];
+      }
+      for (int r = lane + 256; r < n2; r += 64) s += vr[r] * zj[r * zi];
+      s = t * wave_sum(s);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int r = lane + 64 * q;
+        if (r < n2) zj[r * zi] = x[q] - s * v[q];
+      }
+      for (int r = lane + 256; r < n2; r += 64) zj[r * zi] -= s * vr[r];
+      wave_lds_fence();
+    }
+  }
+}
+
+__device__ __noinline__ void syevx_tridiag_vectors(int l, int nev, double* __restrict__ evals,
+                                                   char* __restrict__ ws, double* sv, double* sp, double* sh,
+                                                   double* s_bnd, int cap, double* stg);
+
+// Lowest nev eigenpairs of the symmetric l x l matrix A (leading dim ld), one
+// workgroup: Householder tridiagonalisation, Sturm bisection, inverse
+// iteration (clusters re-orthogonalised), back-transformation.  sv, sp: LDS
+// scratch of cap >= l doubles each; sh: >= blockDim/64 doubles; s_bnd: 2; stg:
+// EIG_STAGE_WAVES * EIG_STAGE doubles of LDS; wl: nl x (nl | 1) doubles of LDS.
+// The reduction runs on global memory until nl rows are left and on LDS from there, the
+// back-transformation on LDS where l nev doubles fit.  In the ensemble (l up to 250, 17 solves
+// of a C22H24 member) with everything on L2 and a row or an element at a time it took 61 ms,
+// now 42: 20 in the steps on L2, 6 on LDS, 13 for the eigenpairs of T, 2 back.
+__device__ __noinline__ void syevx_block(const double* __restrict__ A, int l, int ld, int nev,
+                                         double* __restrict__ evals, double* __restrict__ evecs,
+                                         char* __restrict__ ws, double* sv, double* sp, double* sh, double* s_bnd,
+                                         int cap, double* stg, double* wl, int nl) {
+  EigLayout Lo = eig_layout(l, nev);
+  double* W = (double*)(ws + Lo.W);
+  double* d = (double*)(ws + Lo.d);
+  double* e = (double*)(ws + Lo.e);
+  double* tau = (double*)(ws + Lo.tau);
+  double* Z = (double*)(ws + Lo.z);
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nw = blockDim.x >> 6;
+  lds_f64 *lv = (lds_f64*)sv, *lp = (lds_f64*)sp, *X = (lds_f64*)wl;
+
+  const int j0 = l > nl ? l - nl : 0, ldx = (l - j0) | 1;
+  for (int r = wv; r < l; r += nw)
+    for (int c = lane; c < l; c += 64) {
+      const double a = 0.5 * (A[(long)r * ld + c] + A[(long)c * ld + r]);
+      if (j0 > 0)
+        W[(long)r * l + c] = a;
+      else
+        X[r * ldx + c] = a;
+    }
+  __syncthreads();
+  if (j0 > 0) {
+    hh_block_steps<8, 4>(W, l, 0, j0, l, W, d, e, tau, lv, lp, sh);
+    for (int r = j0 + wv; r < l; r += nw)
+      for (int c = j0 + lane; c < l; c += 64) X[(r - j0) * ldx + (c - j0)] = W[(long)r * l + c];
+    __syncthreads();
+  }
+  if (l > 2) hh_block_steps<4, 2>(X, ldx, j0, l - 2, l, W, d, e, tau, lv, lp, sh);
+  // the last 2 x 2 block
+  if (tid < 4) {
+    const int r = l - 1 - (tid >> 1), c = l - 1 - (tid & 1);
+    if (r >= j0 && c >= j0) W[(long)r * l + c] = X[(r - j0) * ldx + (c - j0)];
+  }
+  __syncthreads();
+  syevx_tridiag_vectors(l, nev, evals, ws, sv, sp, sh, s_bnd, cap, stg);
+  if ((long)l * nev <= (long)nl * (nl | 1)) {
+    for (int i = tid; i < l * nev; i += blockDim.x) {
+      const int r = (unsigned)i / (unsigned)nev;
+      X[(i - r * nev) * l + r] = Z[i];
+    }
+    __syncthreads();
+    hh_block_back(l, nev, W, tau, X, 1, l);
+    __syncthreads();
+    for (int i = tid; i < l * nev; i += blockDim.x) {
+      const int r = (unsigned)i / (unsigned)nev;
+      evecs[i] = X[(i - r * nev) * l + r];
+    }
+  } else {
+    hh_block_back(l, nev, W, tau, Z, nev, 1);
+    __syncthreads();
+    for (int i = tid; i < l * nev; i += blockDim.x) evecs[i] = Z[i];
+  }
 }
 
 // Steps after the Householder reduction of W (reflectors below the first
@@ -684,11 +835,4 @@ __device__ __noinline__ void syevx_back_block(int l, int nev, double* __restrict
     __syncthreads();
   }
   for (long i = tid; i < (long)l * nev; i += blockDim.x) evecs[i] = Z[i];
-}
-
-__device__ __noinline__ void syevx_tail(int l, int nev, double* __restrict__ evals, double* __restrict__ evecs,
-                                        char* __restrict__ ws, int* __restrict__ info, double* sv, double* sp,
-                                        double* sh, double* s_bnd, int cap, double* stg) {
-  syevx_tridiag_vectors(l, nev, evals, ws, sv, sp, sh, s_bnd, cap, stg);
-  syevx_back_block(l, nev, evecs, ws, sv);
 }

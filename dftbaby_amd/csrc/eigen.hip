@@ -31,13 +31,14 @@ extern "C" size_t dftb_syevx_workspace(int l, int nev) { return eig_layout(l, ne
 
 __global__ __launch_bounds__(EIG_THREADS) void syevx_kernel(const double* __restrict__ A, int l, int ld, int nev,
                                                              double* __restrict__ evals, double* __restrict__ evecs,
-                                                             char* __restrict__ ws, int* __restrict__ info) {
+                                                             char* __restrict__ ws) {
   __shared__ double sv[EIG_MAXL];
   __shared__ double sp[EIG_MAXL];
   __shared__ double sh[EIG_THREADS / 64];
   __shared__ double s_bnd[2];
   __shared__ double stg[EIG_STAGE_WAVES * EIG_STAGE];
-  syevx_block(A, l, ld, nev, evals, evecs, ws, info, sv, sp, sh, s_bnd, EIG_MAXL, stg);
+  __shared__ double wl[(EIG_MULTI_L - 1) * (EIG_MULTI_L - 1)];
+  syevx_block(A, l, ld, nev, evals, evecs, ws, sv, sp, sh, s_bnd, EIG_MAXL, stg, wl, EIG_MULTI_L - 1);
 }
 
 // ---- multi-workgroup Householder reduction (large l) -----------------------
@@ -462,8 +463,7 @@ extern "C" int dftb_syevx(const double* A, int l, int ld, int nev, double* evals
   hipStream_t st = (hipStream_t)stream;
   char* ws = (char*)workspace;
   if (l < EIG_MULTI_L) {
-    hipLaunchKernelGGL(syevx_kernel, dim3(1), dim3(EIG_THREADS), 0, st, A, l, ld, nev, evals, evecs, ws,
-                       (int*)nullptr);
+    hipLaunchKernelGGL(syevx_kernel, dim3(1), dim3(EIG_THREADS), 0, st, A, l, ld, nev, evals, evecs, ws);
     DFTB_CHECK_LAUNCH();
     return DFTB_OK;
   }

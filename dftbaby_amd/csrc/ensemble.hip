@@ -1,6 +1,6 @@
 // Persistent ensemble solver: many molecules of uneven size, one launch.
 //
-// Each workgroup runs the complete non-Hermitian Davidson loop of
+// One workgroup per molecule (with helpers, below) runs the complete non-Hermitian Davidson loop of
 // DFTB/Solver.py:637-917 for one molecule on the device (no host round trip
 // per iteration): MFMA matvecs on the molecule's own charges, subspace
 // matrices, Newton-Schulz sqrtm(Mm), the lowest-root eigensolver, residuals,
@@ -15,7 +15,10 @@
 
 #define ENS_THREADS 512
 #define ENS_MAXL 1024   // largest subspace (LDS scratch of the eigensolver)
+#define ENS_EIG_LDS 120  // rows of the eigensolver's matrix in LDS (with the other buffers 154 of 160 KB)
 #define ENS_MAXK 32     // largest number of states
+#define ENS_BLOCKS 8    // most blocks per molecule
+#define ENS_GRID 192    // most blocks of a launch with helpers
 
 // --------------------------------------------------------------------------
 // block-level MFMA GEMM on global operands
@@ -27,7 +30,7 @@
 // so the tile shape does not show in the results.  One CU sustains 614 GFLOP/s in FP32 and
 // 307 in FP64; latency of the loads bounds these products.  With 32 x 32 tiles loaded and
 // multiplied in turn the block products of a C22H24 member (FP32 exchange, 17 iterations) took
-// 188 ms and its Newton-Schulz products 91 ms; with these tiles 127 and 82 ms.
+// 188 ms of one block and its Newton-Schulz products 91 ms; with these tiles 127 and 82 ms.
 // --------------------------------------------------------------------------
 typedef double ens_d2 __attribute__((ext_vector_type(2), aligned(8)));
 typedef float ens_f2 __attribute__((ext_vector_type(2), aligned(4)));
@@ -110,13 +113,13 @@ struct EnsFrag {
 template <typename T, typename TC, int TM, int TN, int KS, bool AT, bool BT>
 __device__ __forceinline__ void bgemm_tiles(int M, int N, int K, const T* __restrict__ A, long lda,
                                             const T* __restrict__ B, long ldb, TC* __restrict__ C, long ldc,
-                                            double alpha, double beta, long cdiv, long cstr) {
+                                            double alpha, double beta, long cdiv, long cstr, int t0, int t1) {
   const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
   const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int tm = (M + 16 * TM - 1) / (16 * TM), tn = (N + 16 * TN - 1) / (16 * TN);
+  const int tn = (N + 16 * TN - 1) / (16 * TN);
   constexpr bool F64 = sizeof(T) == 8;
   const int ns = K / (16 * KS);
-  for (int t = wv; t < tm * tn; t += nw) {
+  for (int t = t0 + wv; t < t1; t += nw) {
     const int m0 = (t / tn) * 16 * TM, n0 = (t % tn) * 16 * TN;
     EnsFrag<T, TM, KS, !AT> fa;
     EnsFrag<T, TN, KS, BT> fb;
@@ -200,53 +203,220 @@ __device__ __forceinline__ void bgemm_tiles(int M, int N, int K, const T* __rest
   }
 }
 
-// cycles of the product over the eight waves (two per SIMD) with TM x TN tiles: MFMA time of
-// a SIMD, operands at about 40 bytes per cycle and CU, or memory latency per buffer
-__device__ __forceinline__ float bgemm_cost(int M, int N, int K, int tm, int tn, int ks, int esz) {
-  const int nt = ((M + 16 * tm - 1) / (16 * tm)) * ((N + 16 * tn - 1) / (16 * tn));
-  const int act = nt < 8 ? nt : 8;
+// tiles of an M x N result
+__device__ __forceinline__ int bgemm_count(int M, int N, int tm, int tn) {
+  return ((M + 16 * tm - 1) / (16 * tm)) * ((N + 16 * tn - 1) / (16 * tn));
+}
+
+// tiles of an item where nb blocks share nt of them: few tiles go to as many blocks as there
+// are, since the operand loads of a block's waves add up
+__device__ __forceinline__ int bgemm_share(int nt, int nb) {
+  const int g = (nt + nb - 1) / nb;
+  return g < 8 ? g : 8;
+}
+
+// cycles of the product over the eight waves (two per SIMD) of nb blocks with TM x TN tiles:
+// MFMA time of a SIMD, operands at about 40 bytes per cycle and CU, or memory latency per buffer
+__device__ __forceinline__ float bgemm_cost(int M, int N, int K, int tm, int tn, int ks, int esz, int nb) {
+  const int nt = bgemm_count(M, N, tm, tn);
+  const int act = bgemm_share(nt, nb);
   const float mf = (esz == 8 ? 256.0f : 128.0f) * tm * tn, op = act * (tm + tn) * 256.0f * esz / 40.0f;
   float w = (act > 4 ? 2.0f : 1.0f) * mf;
   w = fmaxf(w, fmaxf(op, mf + 500.0f / ks));
-  return ((nt + 7) / 8) * (((K + 15) / 16) * w + 1500.0f + 60.0f * tm * tn);
+  return ((nt + act * nb - 1) / (act * nb)) * (((K + 15) / 16) * w + 1500.0f + 60.0f * tm * tn);
 }
 
+// The cheapest tile over nb blocks (0: 16 x 16, 1: 16 x 32, 2: 32 x 32, 3: 32 x 64), its cost and
+// how many of them there are.
+__device__ __forceinline__ int bgemm_pick(int M, int N, int K, int esz, int nb, float* cost, int* nt) {
+  const int kb = esz == 8 ? 2 : 4;            // chunks per buffer of the 32 x 32 tile
+  const float c11 = bgemm_cost(M, N, K, 1, 1, 4, esz, nb), c12 = bgemm_cost(M, N, K, 1, 2, kb, esz, nb);
+  const float c22 = bgemm_cost(M, N, K, 2, 2, kb, esz, nb), c24 = bgemm_cost(M, N, K, 2, 4, kb / 2, esz, nb);
+  const float best = fminf(fminf(c11, c12), fminf(c22, c24));
+  const int tile = best == c24 ? 3 : best == c22 ? 2 : best == c12 ? 1 : 0;
+  *cost = best;
+  *nt = bgemm_count(M, N, tile < 2 ? 1 : 2, tile == 0 ? 1 : tile == 3 ? 4 : 2);
+  return tile;
+}
+
+// tiles t0 <= t < t1 of the product
 template <typename T, typename TC, bool AT, bool BT>
 __device__ __noinline__ void bgemm_t(int M, int N, int K, const T* __restrict__ A, long lda, const T* __restrict__ B,
                                      long ldb, TC* __restrict__ C, long ldc, double alpha, double beta, long cdiv,
-                                     long cstr) {
-  constexpr int E = sizeof(T);
-  constexpr int KB = E == 8 ? 2 : 4;          // chunks per buffer of the 32 x 32 tile
-  const float c11 = bgemm_cost(M, N, K, 1, 1, 4, E), c12 = bgemm_cost(M, N, K, 1, 2, KB, E);
-  const float c22 = bgemm_cost(M, N, K, 2, 2, KB, E), c24 = bgemm_cost(M, N, K, 2, 4, KB / 2, E);
-  const float best = fminf(fminf(c11, c12), fminf(c22, c24));
-  if (best == c24)
-    bgemm_tiles<T, TC, 2, 4, KB / 2, AT, BT>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr);
-  else if (best == c22)
-    bgemm_tiles<T, TC, 2, 2, KB, AT, BT>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr);
-  else if (best == c12)
-    bgemm_tiles<T, TC, 1, 2, KB, AT, BT>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr);
+                                     long cstr, int tile, int t0, int t1) {
+  constexpr int KB = sizeof(T) == 8 ? 2 : 4;
+  if (tile == 3)
+    bgemm_tiles<T, TC, 2, 4, KB / 2, AT, BT>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr, t0, t1);
+  else if (tile == 2)
+    bgemm_tiles<T, TC, 2, 2, KB, AT, BT>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr, t0, t1);
+  else if (tile == 1)
+    bgemm_tiles<T, TC, 1, 2, KB, AT, BT>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr, t0, t1);
   else
-    bgemm_tiles<T, TC, 1, 1, 4, AT, BT>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr);
-  __syncthreads();
+    bgemm_tiles<T, TC, 1, 1, 4, AT, BT>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr, t0, t1);
 }
 
+// the three operand orders in use
+template <typename T, typename TC>
+__device__ __forceinline__ void bgemm_range(int M, int N, int K, const T* A, long lda, int at, const T* B, long ldb,
+                                            int bt, TC* C, long ldc, double alpha, double beta, long cdiv, long cstr,
+                                            int tile, int t0, int t1) {
+  if (at)
+    bgemm_t<T, TC, true, false>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr, tile, t0, t1);
+  else if (bt)
+    bgemm_t<T, TC, false, true>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr, tile, t0, t1);
+  else
+    bgemm_t<T, TC, false, false>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr, tile, t0, t1);
+}
+
+// by this block alone
 template <typename T, typename TC>
 __device__ __forceinline__ void bgemm(int M, int N, int K, const T* A, long lda, int at, const T* B, long ldb, int bt,
                                       TC* C, long ldc, double alpha, double beta, long cdiv, long cstr) {
-  // the three operand orders in use (constant at every call)
-  if (at)
-    bgemm_t<T, TC, true, false>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr);
-  else if (bt)
-    bgemm_t<T, TC, false, true>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr);
-  else
-    bgemm_t<T, TC, false, false>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, cdiv, cstr);
+  float cost;
+  int nt;
+  const int tile = bgemm_pick(M, N, K, sizeof(T), 1, &cost, &nt);
+  bgemm_range<T, TC>(M, N, K, A, lda, at, B, ldb, bt, C, ldc, alpha, beta, cdiv, cstr, tile, 0, nt);
+  __syncthreads();
 }
 
-template <typename T, typename TC>
-__device__ __forceinline__ void bg(int M, int N, int K, const T* A, long lda, int at, const T* B, long ldb, int bt,
-                                   TC* C, long ldc, double alpha = 1.0, double beta = 0.0) {
-  bgemm<T, TC>(M, N, K, A, lda, at, B, ldb, bt, C, ldc, alpha, beta, 0, 0);
+// --------------------------------------------------------------------------
+// Work shared between the blocks of a molecule.
+// One block, the leader, runs the molecule's loop.  The large products and the exchange of a
+// block of vectors are cut into items that its helpers (further blocks of the launch) take
+// along with the leader, by tickets; the items are the same whoever takes them.  Nothing waits
+// for a block that may not be running: the leader takes every item that no helper has taken and
+// then waits only for items that running helpers hold; a helper whose leader has not started
+// within 0.2 ms ends, and the others end when the leader says so.
+// 24 members on one block each leave nine tenths of the chip idle: with up to eight blocks each
+// 24 polyenes C8-C22 (8 states, FP32 exchange) take 131 ms instead of 326; of a C22H24 member's
+// time the block products fell from 127 to 19 ms, the matrix square roots from 82 to 33.
+// --------------------------------------------------------------------------
+#define ENS_ITEM_BITS 24
+#define ENS_STARTED (1ull << 62)
+#define ENS_QUIT (1ull << 63)
+
+struct EnsProduct {                        // C = alpha op(A) op(B) + beta C
+  int M, N, K, at, bt;
+  const double* A;
+  long lda;
+  const double* B;
+  long ldb;
+  double* C;
+  long ldc;
+  double alpha, beta;
+  int tile, nt, share, end;                // tile shape, tiles, tiles per item, items up to here
+};
+
+#define ENS_PRODUCTS 4
+struct EnsTask {
+  int np;                                  // products; 0: the exchange of a block of vectors
+  EnsProduct p[ENS_PRODUCTS];
+  const double* V;
+  double *outP, *outM;
+};
+
+struct EnsCtl {
+  unsigned long long word;                 // flags, items of the current section, next item
+  char pad0[120];
+  unsigned long long done;                 // items finished by helpers since the launch began
+  char pad1[120];
+  EnsTask task;
+};
+
+struct EnsShare {                          // the leader's view
+  EnsCtl* ctl;
+  int nb;                                  // blocks of this molecule
+  int* s_item;                             // LDS
+  unsigned long long done;                 // items that helpers have finished so far
+};
+
+__device__ __forceinline__ unsigned long long ens_load(const unsigned long long* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// next item of the current section, or -1.  One thread's fences and the barriers around them
+// order the accesses of the whole block.
+template <bool HELPER>
+__device__ __forceinline__ int ens_take(EnsCtl* ctl, int* s_item) {
+  if (threadIdx.x == 0) {
+    const unsigned long long old =
+        __hip_atomic_fetch_add(&ctl->word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long mask = (1ull << ENS_ITEM_BITS) - 1, idx = old & mask;
+    *s_item = (old & ENS_QUIT) || idx >= ((old >> ENS_ITEM_BITS) & mask) ? -1 : (int)idx;
+    if (HELPER) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  }
+  __syncthreads();
+  const int item = *s_item;
+  __syncthreads();
+  return item;
+}
+
+template <typename F>
+__device__ __forceinline__ void ens_section(EnsShare& sh, int items, F&& run) {
+  // thread 0 has written the task
+  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(&sh.ctl->word, ENS_STARTED | ((unsigned long long)items << ENS_ITEM_BITS), __ATOMIC_RELEASE,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  int mine = 0;
+  for (int i = ens_take<false>(sh.ctl, sh.s_item); i >= 0; i = ens_take<false>(sh.ctl, sh.s_item)) {
+    run(i);
+    ++mine;
+  }
+  sh.done += items - mine;
+  if (threadIdx.x == 0) {
+    while (ens_load(&sh.ctl->done) != sh.done) __builtin_amdgcn_s_sleep(1);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  }
+  __syncthreads();
+}
+
+// item i of a section of products
+__device__ __noinline__ void ens_product_item(const EnsTask* t, int i) {
+  int q = 0;
+  while (i >= t->p[q].end) ++q;
+  const EnsProduct& p = t->p[q];
+  const int t0 = (i - (q > 0 ? t->p[q - 1].end : 0)) * p.share;
+  bgemm_range<double, double>(p.M, p.N, p.K, p.A, p.lda, p.at, p.B, p.ldb, p.bt, p.C, p.ldc, p.alpha, p.beta, 0, 0,
+                              p.tile, t0, t0 + p.share < p.nt ? t0 + p.share : p.nt);
+}
+
+// Independent products, by all blocks of the molecule where the estimate for them, with 12000
+// cycles for handing a section out and collecting it, is the lower one.
+template <int NP>
+__device__ __noinline__ void pg(EnsShare& sh, EnsProduct (&p)[NP]) {
+  float c1 = 0.0f, cn = 0.0f;
+  int items = 0, t1[NP], n1[NP];
+  for (int q = 0; q < NP; ++q) {
+    float c;
+    t1[q] = bgemm_pick(p[q].M, p[q].N, p[q].K, 8, 1, &c, &n1[q]);
+    c1 += c;
+    p[q].tile = bgemm_pick(p[q].M, p[q].N, p[q].K, 8, sh.nb, &c, &p[q].nt);
+    cn += c;
+    p[q].share = bgemm_share(p[q].nt, sh.nb);
+    items += (p[q].nt + p[q].share - 1) / p[q].share;
+    p[q].end = items;
+  }
+  if (sh.nb > 1 && cn + 12000.0f < c1) {
+    EnsTask* t = &sh.ctl->task;
+    if (threadIdx.x == 0) {
+      t->np = NP;
+      for (int q = 0; q < NP; ++q) t->p[q] = p[q];
+    }
+    ens_section(sh, items, [&](int i) { ens_product_item(t, i); });
+  } else {
+    for (int q = 0; q < NP; ++q)
+      bgemm_range<double, double>(p[q].M, p[q].N, p[q].K, p[q].A, p[q].lda, p[q].at, p[q].B, p[q].ldb, p[q].bt,
+                                  p[q].C, p[q].ldc, p[q].alpha, p[q].beta, 0, 0, t1[q], 0, n1[q]);
+    __syncthreads();
+  }
+}
+
+__device__ __forceinline__ void pg(EnsShare& sh, int M, int N, int K, const double* A, long lda, int at,
+                                   const double* B, long ldb, int bt, double* C, long ldc, double alpha = 1.0,
+                                   double beta = 0.0) {
+  EnsProduct p[1] = {{M, N, K, at, bt, A, lda, B, ldb, C, ldc, alpha, beta, 0, 0, 0, 0}};
+  pg(sh, p);
 }
 
 __device__ double bsum(double v, double* sh) {
@@ -275,8 +445,9 @@ __device__ double bmax(double v, double* sh) {
 // per-molecule workspace layout (host and device agree)
 // --------------------------------------------------------------------------
 struct EnsLayout {
-  size_t TT, X1, X2, tv, gv, Sq, Sinv, H, Y2, Z2, P, Tns, eig, Tbv, Rb, Lb, R, L, PR, ML, W, nrm, w2, G, Lc, Li, ref,
-      Qt, v32, keep, total;
+  size_t TT, X1, X2, tv, gv, Sq, Sinv, H, Y2, Z2, P, Tns, eig, Tbv, Rb, Lb, R, L, PR, ML, W, nrm, w2, G, Li, ref,
+      Qt, v32, keep, ctl, tt, total;
+  int slots;  // blocks that have an expansion buffer TT
 };
 
 __host__ __device__ static long ens_mmax(const EnsMolecule& m) {
@@ -290,19 +461,23 @@ __host__ __device__ static EnsLayout ens_layout(const EnsMolecule& m) {
   const long rows = m.opad > m.vpad ? m.opad : m.vpad;
   const long mm = ens_mmax(m);
   const long cap = m.cap, k = m.k;
+  // one TT per block while they stay within 256 MB
+  L.tt = al256((size_t)m.nat * rows * m.vpad * 8);
+  const size_t fit = ((size_t)1 << 28) / L.tt;
+  L.slots = fit < 1 ? 1 : fit > ENS_BLOCKS ? ENS_BLOCKS : (int)fit;
   size_t o = 0;
   size_t* fields[] = {&L.TT, &L.X1, &L.X2, &L.tv, &L.gv, &L.Sq, &L.Sinv, &L.H, &L.Y2, &L.Z2, &L.P, &L.Tns, &L.eig,
-                      &L.Tbv, &L.Rb, &L.Lb, &L.R, &L.L, &L.PR, &L.ML, &L.W, &L.nrm, &L.w2, &L.G, &L.Lc, &L.Li,
-                      &L.ref, &L.Qt, &L.v32, &L.keep};
-  const size_t sizes[] = {(size_t)m.nat * rows * m.vpad * 8, (size_t)mm * N * 8, (size_t)mm * N * 8,
+                      &L.Tbv, &L.Rb, &L.Lb, &L.R, &L.L, &L.PR, &L.ML, &L.W, &L.nrm, &L.w2, &L.G, &L.Li,
+                      &L.ref, &L.Qt, &L.v32, &L.keep, &L.ctl};
+  const size_t sizes[] = {L.tt * L.slots, (size_t)mm * N * 8, (size_t)mm * N * 8,
                           (size_t)mm * m.nat * 8, (size_t)mm * m.nat * 8, (size_t)cap * cap * 8,
                           (size_t)cap * cap * 8, (size_t)cap * cap * 8, (size_t)cap * cap * 8,
                           (size_t)cap * cap * 8, (size_t)cap * cap * 8, (size_t)cap * cap * 8,
                           eig_layout((int)cap, (int)k).total, (size_t)cap * k * 8, (size_t)cap * k * 8,
                           (size_t)cap * k * 8, (size_t)k * N * 8, (size_t)k * N * 8, (size_t)k * N * 8,
                           (size_t)k * N * 8, (size_t)2 * k * N * 8, (size_t)2 * k * 8, (size_t)k * 8,
-                          (size_t)mm * mm * 8, (size_t)mm * mm * 8, (size_t)mm * mm * 8, (size_t)mm * 8,
-                          (size_t)mm * N * 8, (size_t)mm * N * 4, (size_t)mm * 4};
+                          (size_t)mm * mm * 8, (size_t)mm * mm * 8, (size_t)mm * 8,
+                          (size_t)mm * N * 8, (size_t)mm * N * 4, (size_t)mm * 4, sizeof(EnsCtl)};
   for (int i = 0; i < 30; ++i) {
     *fields[i] = o;
     o += al256(sizes[i]);
@@ -316,74 +491,133 @@ extern "C" size_t dftb_ensemble_workspace(const EnsMolecule* m) { return ens_lay
 // --------------------------------------------------------------------------
 // matvec of m vectors V (FP64, [m][N]) -> outP = (A+B)V, outM = (A-B)V
 // --------------------------------------------------------------------------
+// vector n: the exchange and the sum, in the buffer TT of the block that does it; outP holds the
+// Coulomb part
 template <typename T>
-__device__ void ens_matvec(const EnsMolecule& Mo, char* ws, const EnsLayout& L, const double* Vd, int m, double* outP,
-                           double* outM) {
-  const long N = (long)Mo.opad * Mo.vpad, nat = Mo.nat, op = Mo.opad, vp = Mo.vpad;
-  double* tv = (double*)(ws + L.tv);
-  double* gv = (double*)(ws + L.gv);
-  double* X1 = (double*)(ws + L.X1);
-  double* X2 = (double*)(ws + L.X2);
-  const long total = (long)m * N;
-  // Coulomb: t = V q_c^T, g = t gamma, outP = 4 g q_c  (FP64)
-  bg<double, double>(m, (int)nat, (int)N, Vd, N, 0, Mo.q_c, N, 1, tv, nat);
-  bg<double, double>(m, (int)nat, (int)nat, tv, nat, 0, Mo.gamma, nat, 0, gv, nat);
-  bg<double, double>(m, (int)N, (int)nat, gv, nat, 0, Mo.q_c, N, 0, outP, N, 4.0, 0.0);
-  if (Mo.lc) {
-    for (long i = threadIdx.x; i < total; i += blockDim.x) {
-      X1[i] = 0.0;
-      X2[i] = 0.0;
-    }
-    const T* V = (const T*)Vd;
-    if (sizeof(T) == 4) {
-      float* v32 = (float*)(ws + L.v32);
-      for (long i = threadIdx.x; i < total; i += blockDim.x) v32[i] = (float)Vd[i];
-      V = (const T*)v32;
-    }
-    __syncthreads();
-    const T* qoo = (const T*)(sizeof(T) == 4 ? Mo.q32[0] : Mo.q_oo);
-    const T* qov = (const T*)(sizeof(T) == 4 ? Mo.q32[1] : Mo.q_ov);
-    const T* qfov = (const T*)(sizeof(T) == 4 ? Mo.q32[2] : Mo.qf_ov);
-    const T* qfvv = (const T*)(sizeof(T) == 4 ? Mo.q32[3] : Mo.qf_vv);
-    T* TT = (T*)(ws + L.TT);
-    for (int n = 0; n < m; ++n) {
-      const T* v = V + (long)n * N;
-      // K1 expand: T[A][j][a] = sum_b V[j][b] qf_vv[b][A][a]
-      bgemm<T, T>((int)op, (int)(nat * vp), (int)vp, v, vp, 0, qfvv, nat * vp, 0, TT, vp, 1.0, 0.0, vp, op * vp);
-      // K1 contract: X1[i][a] = sum_{A,j} q_oo[i][A][j] T[A][j][a]
-      bgemm<T, double>(Mo.nocc, (int)vp, (int)(nat * op), qoo, nat * op, 0, TT, vp, 0, X1 + (long)n * N, vp, 1.0, 0.0,
-                       0, 0);
-      // K2 expand: U[A][b][a] = sum_j V[j][b] qf_ov[j][A][a]
-      bgemm<T, T>((int)vp, (int)(nat * vp), Mo.nocc, v, vp, 1, qfov, nat * vp, 0, TT, vp, 1.0, 0.0, vp, vp * vp);
-      // K2 contract: X2[i][a] = sum_{A,b} q_ov[i][A][b] U[A][b][a]
-      bgemm<T, double>(Mo.nocc, (int)vp, (int)(nat * vp), qov, nat * vp, 0, TT, vp, 0, X2 + (long)n * N, vp, 1.0, 0.0,
-                       0, 0);
-    }
+__device__ __noinline__ void ens_exchange(const EnsMolecule& Mo, char* ws, const EnsLayout& L, int slot,
+                                          const double* Vd, int n, double* outP, double* outM) {
+  const long N = (long)Mo.opad * Mo.vpad, nat = Mo.nat, op = Mo.opad, vp = Mo.vpad, o = n * N;
+  double* X1 = (double*)(ws + L.X1) + o;
+  double* X2 = (double*)(ws + L.X2) + o;
+  for (long i = threadIdx.x; i < N; i += blockDim.x) {
+    X1[i] = 0.0;
+    X2[i] = 0.0;
   }
-  for (long i = threadIdx.x; i < total; i += blockDim.x) {
-    const long e = i % N;
-    const double ov = Mo.omega[e] * Vd[i];
-    const double k1 = Mo.lc ? X1[i] : 0.0, k2 = Mo.lc ? X2[i] : 0.0;
-    outP[i] = ov + outP[i] - k1 - k2;
-    outM[i] = ov - k1 + k2;
+  const T* v = (const T*)Vd + o;
+  if (sizeof(T) == 4) {
+    float* v32 = (float*)(ws + L.v32) + o;
+    for (long i = threadIdx.x; i < N; i += blockDim.x) v32[i] = (float)Vd[o + i];
+    v = (const T*)v32;
+  }
+  __syncthreads();
+  const T* qoo = (const T*)(sizeof(T) == 4 ? Mo.q32[0] : Mo.q_oo);
+  const T* qov = (const T*)(sizeof(T) == 4 ? Mo.q32[1] : Mo.q_ov);
+  const T* qfov = (const T*)(sizeof(T) == 4 ? Mo.q32[2] : Mo.qf_ov);
+  const T* qfvv = (const T*)(sizeof(T) == 4 ? Mo.q32[3] : Mo.qf_vv);
+  T* TT = (T*)(ws + L.TT + slot * L.tt);
+  // K1 expand: T[A][j][a] = sum_b V[j][b] qf_vv[b][A][a]
+  bgemm<T, T>((int)op, (int)(nat * vp), (int)vp, v, vp, 0, qfvv, nat * vp, 0, TT, vp, 1.0, 0.0, vp, op * vp);
+  // K1 contract: X1[i][a] = sum_{A,j} q_oo[i][A][j] T[A][j][a]
+  bgemm<T, double>(Mo.nocc, (int)vp, (int)(nat * op), qoo, nat * op, 0, TT, vp, 0, X1, vp, 1.0, 0.0, 0, 0);
+  // K2 expand: U[A][b][a] = sum_j V[j][b] qf_ov[j][A][a]
+  bgemm<T, T>((int)vp, (int)(nat * vp), Mo.nocc, v, vp, 1, qfov, nat * vp, 0, TT, vp, 1.0, 0.0, vp, vp * vp);
+  // K2 contract: X2[i][a] = sum_{A,b} q_ov[i][A][b] U[A][b][a]
+  bgemm<T, double>(Mo.nocc, (int)vp, (int)(nat * vp), qov, nat * vp, 0, TT, vp, 0, X2, vp, 1.0, 0.0, 0, 0);
+  for (long i = threadIdx.x; i < N; i += blockDim.x) {
+    const double ov = Mo.omega[i] * Vd[o + i];
+    const double k1 = X1[i], k2 = X2[i];
+    outP[o + i] = ov + outP[o + i] - k1 - k2;
+    outM[o + i] = ov - k1 + k2;
   }
   __syncthreads();
 }
 
-// --------------------------------------------------------------------------
-// Newton-Schulz sqrt of the l x l block of A (ld): S = A^{1/2}, Si = A^{-1/2}
-// returns 0 on success, nonzero if not converged (A not positive definite)
-// --------------------------------------------------------------------------
-__device__ int ens_sqrtm(const double* A, int l, int ld, double* S, double* Si, double* T, double* P, double* Y2,
-                         double* Z2, double* sh) {
+template <typename T>
+__device__ void ens_matvec(EnsShare& sh, const EnsMolecule& Mo, char* ws, const EnsLayout& L, const double* Vd, int m,
+                           double* outP, double* outM) {
+  const long N = (long)Mo.opad * Mo.vpad, nat = Mo.nat;
+  double* tv = (double*)(ws + L.tv);
+  double* gv = (double*)(ws + L.gv);
+  // Coulomb: t = V q_c^T, g = t gamma, outP = 4 g q_c  (FP64)
+  pg(sh, m, (int)nat, (int)N, Vd, N, 0, Mo.q_c, N, 1, tv, nat);
+  pg(sh, m, (int)nat, (int)nat, tv, nat, 0, Mo.gamma, nat, 0, gv, nat);
+  pg(sh, m, (int)N, (int)nat, gv, nat, 0, Mo.q_c, N, 0, outP, N, 4.0, 0.0);
+  if (Mo.lc) {
+    if (sh.nb > 1 && m > 1) {
+      if (threadIdx.x == 0) {
+        EnsTask* t = &sh.ctl->task;
+        t->np = 0;
+        t->V = Vd;
+        t->outP = outP;
+        t->outM = outM;
+      }
+      ens_section(sh, m, [&](int n) { ens_exchange<T>(Mo, ws, L, 0, Vd, n, outP, outM); });
+    } else {
+      for (int n = 0; n < m; ++n) ens_exchange<T>(Mo, ws, L, 0, Vd, n, outP, outM);
+    }
+    return;
+  }
+  for (int n = 0; n < m; ++n)
+    for (long i = threadIdx.x; i < N; i += blockDim.x) {
+      const double ov = Mo.omega[i] * Vd[n * N + i];
+      outP[n * N + i] = ov + outP[n * N + i];
+      outM[n * N + i] = ov;
+    }
+  __syncthreads();
+}
+
+// helper number slot of a molecule: items until the leader ends
+template <typename T>
+__device__ void ens_help(const EnsMolecule& Mo, int slot, int* s_item) {
+  char* ws = (char*)Mo.work;
+  const EnsLayout L = ens_layout(Mo);
+  EnsCtl* ctl = (EnsCtl*)(ws + L.ctl);
+  if (slot >= L.slots) return;
+  const unsigned long long mask = (1ull << ENS_ITEM_BITS) - 1;
+  const unsigned long long t0 = wall_clock64();
+  for (;;) {
+    if (threadIdx.x == 0) {
+      // -1: the leader has ended, or did not start within 0.2 ms (100 MHz clock); 1: an item may be free
+      int go = 0;
+      while (!go) {
+        const unsigned long long w = ens_load(&ctl->word);
+        if ((w & ENS_QUIT) || (!(w & ENS_STARTED) && wall_clock64() - t0 > 20000))
+          go = -1;
+        else if ((w & mask) < ((w >> ENS_ITEM_BITS) & mask))
+          go = 1;
+        else
+          __builtin_amdgcn_s_sleep(8);
+      }
+      *s_item = go;
+    }
+    __syncthreads();
+    const int go = *s_item;
+    __syncthreads();
+    if (go < 0) return;
+    const int i = ens_take<true>(ctl, s_item);
+    if (i < 0) continue;
+    const EnsTask* t = &ctl->task;
+    if (t->np == 0)
+      ens_exchange<T>(Mo, ws, L, slot, t->V, i, t->outP, t->outM);
+    else
+      ens_product_item(t, i);
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_fetch_add(&ctl->done, 1ull, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// S = sqrt(A), Si = its inverse; both end in the buffers passed as S and Si
+__device__ int ens_sqrtm(EnsShare& es, const double* A, int l, int ld, double* S, double* Si, double* T, double* P,
+                         double* Y2, double* Z2, double* sh) {
+  double *const S0 = S, *const Si0 = Si;
   double fro = 0.0;
-  for (long i = threadIdx.x; i < (long)l * l; i += blockDim.x) {
-    double a = A[(i / l) * ld + i % l];
+  for (int i = threadIdx.x; i < l * l; i += blockDim.x) {
+    double a = A[(long)((unsigned)i / (unsigned)l) * ld + (unsigned)i % (unsigned)l];
     fro += a * a;
   }
   const double c = fmax(sqrt(bsum(fro, sh)), 1e-300);
-  for (long i = threadIdx.x; i < (long)l * l; i += blockDim.x) {
-    int r = (int)(i / l), q = (int)(i % l);
+  for (int i = threadIdx.x; i < l * l; i += blockDim.x) {
+    const int r = (unsigned)i / (unsigned)l, q = i - r * l;
     S[i] = 0.5 * (A[(long)r * ld + q] + A[(long)q * ld + r]) / c;
     Si[i] = (r == q) ? 1.0 : 0.0;
   }
@@ -391,10 +625,10 @@ __device__ int ens_sqrtm(const double* A, int l, int ld, double* S, double* Si, 
   double err = 1.0;
   int ok = 0;
   for (int it = 0; it < 100; ++it) {
-    bg<double, double>(l, l, l, Si, l, 0, S, l, 0, P, l);
+    pg(es, l, l, l, Si, l, 0, S, l, 0, P, l);
     double m = 0.0;
-    for (long i = threadIdx.x; i < (long)l * l; i += blockDim.x) {
-      int r = (int)(i / l), q = (int)(i % l);
+    for (int i = threadIdx.x; i < l * l; i += blockDim.x) {
+      const int r = (unsigned)i / (unsigned)l, q = i - r * l;
       double id = (r == q) ? 1.0 : 0.0;
       m = fmax(m, fabs(P[i] - id));
       T[i] = 0.5 * (3.0 * id - P[i]);
@@ -405,19 +639,20 @@ __device__ int ens_sqrtm(const double* A, int l, int ld, double* S, double* Si, 
       ok = 1;
       break;
     }
-    bg<double, double>(l, l, l, S, l, 0, T, l, 0, Y2, l);
-    bg<double, double>(l, l, l, T, l, 0, Si, l, 0, Z2, l);
-    for (long i = threadIdx.x; i < (long)l * l; i += blockDim.x) {
-      S[i] = Y2[i];
-      Si[i] = Z2[i];
-    }
-    __syncthreads();
+    EnsProduct yz[2] = {{l, l, l, 0, 0, S, l, T, l, Y2, l, 1.0, 0.0}, {l, l, l, 0, 0, T, l, Si, l, Z2, l, 1.0, 0.0}};
+    pg(es, yz);
+    double* x = S;
+    S = Y2;
+    Y2 = x;
+    x = Si;
+    Si = Z2;
+    Z2 = x;
   }
   if (!ok && err < 1e-10) ok = 1;
   const double f = sqrt(c);
-  for (long i = threadIdx.x; i < (long)l * l; i += blockDim.x) {
-    S[i] *= f;
-    Si[i] /= f;
+  for (int i = threadIdx.x; i < l * l; i += blockDim.x) {
+    S0[i] = S[i] * f;
+    Si0[i] = Si[i] / f;
   }
   __syncthreads();
   return ok ? 0 : 1;
@@ -427,7 +662,7 @@ __device__ int ens_sqrtm(const double* A, int l, int ld, double* S, double* Si, 
 // orthonormalise rows Q[0..m) (N) against B[0..l) and among themselves;
 // dependent rows dropped (compacted); returns the number kept
 // --------------------------------------------------------------------------
-__device__ int ens_orthonormalize(const double* B, int l, double* Q, int m, long N, double tol, double* Cc, double* G,
+__device__ int ens_orthonormalize(EnsShare& es, const double* B, int l, double* Q, int m, long N, double tol, double* Cc, double* G,
                                   double* Lc, double* Li, double* ref, double* Qt, int* keep, double* sh) {
   for (int t = 0; t < m; ++t) {
     double s = 0.0;
@@ -440,47 +675,49 @@ __device__ int ens_orthonormalize(const double* B, int l, double* Q, int m, long
   }
   __syncthreads();
   for (int pass = 0; pass < 2 && l > 0; ++pass) {
-    bg<double, double>(l, m, (int)N, B, N, 0, Q, N, 1, Cc, m);            // Cc[p][t] = <B_p, Q_t>
-    bg<double, double>(m, (int)N, l, Cc, m, 1, B, N, 0, Q, N, -1.0, 1.0);  // Q -= Cc^T B
+    pg(es, l, m, (int)N, B, N, 0, Q, N, 1, Cc, m);            // Cc[p][t] = <B_p, Q_t>
+    pg(es, m, (int)N, l, Cc, m, 1, B, N, 0, Q, N, -1.0, 1.0);  // Q -= Cc^T B
   }
   for (int pass = 0; pass < 2; ++pass) {
-    bg<double, double>(m, m, (int)N, Q, N, 0, Q, N, 1, G, m);
-    for (int i = threadIdx.x; i < m * m; i += blockDim.x) {
-      Lc[i] = 0.0;
-      Li[i] = 0.0;
-    }
+    pg(es, m, m, (int)N, Q, N, 0, Q, N, 1, G, m);
+    // column by column, one row per thread (the factor's rows packed in LDS); then the inverse,
+    // one column per thread
+    for (int i = threadIdx.x; i < m * (m + 1) / 2; i += blockDim.x) Lc[i] = 0.0;
+    for (int i = threadIdx.x; i < m * m; i += blockDim.x) Li[i] = 0.0;
     __syncthreads();
-    // column by column, one row per thread; then the inverse, one column per thread
     for (int j = 0; j < m; ++j) {
+      const double* Lj = Lc + j * (j + 1) / 2;
       if (threadIdx.x == 0) {
         double d = G[j * m + j];
-        for (int q = 0; q < j; ++q) d -= Lc[j * m + q] * Lc[j * m + q];
+        for (int q = 0; q < j; ++q) d -= Lj[q] * Lj[q];
         const double r = pass == 0 ? ref[j] * ref[j] : 1.0;
         const double t2 = pass == 0 ? tol * tol : 1e-24;
         const int ok = keep[j] && d > t2 * r && d > 1e-12 * G[j * m + j] && d > 0.0;
         keep[j] = ok;
-        Lc[j * m + j] = ok ? sqrt(d) : 1.0;
+        Lc[j * (j + 1) / 2 + j] = ok ? sqrt(d) : 1.0;
       }
       __syncthreads();
       if (keep[j])
         for (int i = j + 1 + threadIdx.x; i < m; i += blockDim.x) {
+          double* Lr = Lc + i * (i + 1) / 2;
           double s = G[i * m + j];
-          for (int q = 0; q < j; ++q) s -= Lc[i * m + q] * Lc[j * m + q];
-          Lc[i * m + j] = s / Lc[j * m + j];
+          for (int q = 0; q < j; ++q) s -= Lr[q] * Lj[q];
+          Lr[j] = s / Lj[j];
         }
       __syncthreads();
     }
     for (int c = threadIdx.x; c < m; c += blockDim.x)
       for (int i = c; i < m; ++i) {
+        const double* Lr = Lc + i * (i + 1) / 2;
         double s = (i == c) ? 1.0 : 0.0;
-        for (int q = c; q < i; ++q) s -= Lc[i * m + q] * Li[q * m + c];
-        Li[i * m + c] = s / Lc[i * m + i];
+        for (int q = c; q < i; ++q) s -= Lr[q] * Li[q * m + c];
+        Li[i * m + c] = s / Lr[i];
       }
     __syncthreads();
     for (int i = threadIdx.x; i < m * m; i += blockDim.x)
       if (!keep[i / m]) Li[i] = 0.0;
     __syncthreads();
-    bg<double, double>(m, (int)N, m, Li, m, 0, Q, N, 0, Qt, N);
+    pg(es, m, (int)N, m, Li, m, 0, Q, N, 0, Qt, N);
     for (long i = threadIdx.x; i < (long)m * N; i += blockDim.x) Q[i] = Qt[i];
     __syncthreads();
   }
@@ -502,9 +739,12 @@ __device__ int ens_orthonormalize(const double* B, int l, double* Q, int m, long
 // --------------------------------------------------------------------------
 template <typename T>
 __device__ void ens_davidson(const EnsMolecule& Mo, double conv, int maxiter, double* sh, double* sv, double* sp,
-                             double* bnd, int* s_sel, double* stg) {
+                             double* bnd, int* s_sel, double* stg, double* wl, int nb) {
   char* ws = (char*)Mo.work;
   const EnsLayout L = ens_layout(Mo);
+  EnsShare es = {(EnsCtl*)(ws + L.ctl), nb < L.slots ? nb : L.slots, s_sel + 2 * ENS_MAXK + 1, 0};
+  if (threadIdx.x == 0)
+    __hip_atomic_store(&es.ctl->word, ENS_STARTED, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
   const long N = (long)Mo.opad * Mo.vpad;
   const int k = Mo.k, cap = Mo.cap;
   const long kmax = (long)Mo.nocc * Mo.nvirt;
@@ -539,19 +779,24 @@ __device__ void ens_davidson(const EnsMolecule& Mo, double conv, int maxiter, do
   for (it = 0; it < maxiter; ++it) {
     const int m = l - new0;
     if (m > 0) {
-      ens_matvec<T>(Mo, ws, L, bs + (long)new0 * N, m, bp + (long)new0 * N, bm + (long)new0 * N);
+      ens_matvec<T>(es, Mo, ws, L, bs + (long)new0 * N, m, bp + (long)new0 * N, bm + (long)new0 * N);
       // new columns/rows of M+- = bs^T (A+-B) bs
-      bg<double, double>(l, m, (int)N, bs, N, 0, bp + (long)new0 * N, N, 1, Mp + new0, cap);
-      bg<double, double>(l, m, (int)N, bs, N, 0, bm + (long)new0 * N, N, 1, Mm + new0, cap);
+      const double* bn = bs + (long)new0 * N;
+      EnsProduct cols[2] = {{l, m, (int)N, 0, 1, bs, N, bp + (long)new0 * N, N, Mp + new0, cap, 1.0, 0.0},
+                            {l, m, (int)N, 0, 1, bs, N, bm + (long)new0 * N, N, Mm + new0, cap, 1.0, 0.0}};
       if (new0 > 0) {
-        bg<double, double>(m, new0, (int)N, bs + (long)new0 * N, N, 0, bp, N, 1, Mp + (long)new0 * cap, cap);
-        bg<double, double>(m, new0, (int)N, bs + (long)new0 * N, N, 0, bm, N, 1, Mm + (long)new0 * cap, cap);
+        EnsProduct all[4] = {cols[0], cols[1],
+                             {m, new0, (int)N, 0, 1, bn, N, bp, N, Mp + (long)new0 * cap, cap, 1.0, 0.0},
+                             {m, new0, (int)N, 0, 1, bn, N, bm, N, Mm + (long)new0 * cap, cap, 1.0, 0.0}};
+        pg(es, all);
+      } else {
+        pg(es, cols);
       }
     }
     if (sizeof(T) == 4) {
       // FP32 products: use the symmetric parts of M+-
-      for (long i = threadIdx.x; i < (long)l * l; i += blockDim.x) {
-        int r = (int)(i / l), c = (int)(i % l);
+      for (int i = threadIdx.x; i < l * l; i += blockDim.x) {
+        const int r = (unsigned)i / (unsigned)l, c = i - r * l;
         if (c > r) {
           double a = 0.5 * (Mp[(long)r * cap + c] + Mp[(long)c * cap + r]);
           Mp[(long)r * cap + c] = a;
@@ -564,16 +809,16 @@ __device__ void ens_davidson(const EnsMolecule& Mo, double conv, int maxiter, do
       __syncthreads();
     }
     // subspace step (Solver.py:759-798)
-    if (ens_sqrtm(Mm, l, cap, Sq, Sinv, (double*)(ws + L.Tns), (double*)(ws + L.P), (double*)(ws + L.Y2),
+    if (ens_sqrtm(es, Mm, l, cap, Sq, Sinv, (double*)(ws + L.Tns), (double*)(ws + L.P), (double*)(ws + L.Y2),
                   (double*)(ws + L.Z2), sh)) {
       code = -3;
       break;
     }
-    bg<double, double>(l, l, l, Mp, cap, 0, Sq, l, 0, (double*)(ws + L.P), l);
-    bg<double, double>(l, l, l, Sq, l, 0, (double*)(ws + L.P), l, 0, H, l);
+    pg(es, l, l, l, Mp, cap, 0, Sq, l, 0, (double*)(ws + L.P), l);
+    pg(es, l, l, l, Sq, l, 0, (double*)(ws + L.P), l, 0, H, l);
     double he = 0.0;
-    for (long i = threadIdx.x; i < (long)l * l; i += blockDim.x) {
-      int r = (int)(i / l), c = (int)(i % l);
+    for (int i = threadIdx.x; i < l * l; i += blockDim.x) {
+      const int r = (unsigned)i / (unsigned)l, c = i - r * l;
       he += fabs(H[(long)r * l + c] - H[(long)c * l + r]);
     }
     he = bsum(he, sh);
@@ -582,7 +827,7 @@ __device__ void ens_davidson(const EnsMolecule& Mo, double conv, int maxiter, do
       break;
     }
     const int nev = k < l ? k : l;
-    syevx_block(H, l, l, nev, w2, Tb, ws + L.eig, nullptr, sv, sp, sh, bnd, ENS_MAXL, stg);
+    syevx_block(H, l, l, nev, w2, Tb, ws + L.eig, sv, sp, sh, bnd, ENS_MAXL, stg, wl, ENS_EIG_LDS);
     __syncthreads();
     int bad = 0;
     for (int n = threadIdx.x; n < nev; n += blockDim.x)
@@ -593,17 +838,18 @@ __device__ void ens_davidson(const EnsMolecule& Mo, double conv, int maxiter, do
     }
     for (int n = threadIdx.x; n < nev; n += blockDim.x) w[n] = sqrt(w2[n]);
     __syncthreads();
-    bg<double, double>(l, nev, l, Sq, l, 0, Tb, nev, 0, Rb, nev);
-    for (long i = threadIdx.x; i < (long)l * nev; i += blockDim.x) Rb[i] /= sqrt(w[i % nev]);
+    pg(es, l, nev, l, Sq, l, 0, Tb, nev, 0, Rb, nev);
+    for (int i = threadIdx.x; i < l * nev; i += blockDim.x) Rb[i] /= sqrt(w[(unsigned)i % (unsigned)nev]);
     __syncthreads();
-    bg<double, double>(l, nev, l, Mp, cap, 0, Rb, nev, 0, Lb, nev);
-    for (long i = threadIdx.x; i < (long)l * nev; i += blockDim.x) Lb[i] /= w[i % nev];
+    pg(es, l, nev, l, Mp, cap, 0, Rb, nev, 0, Lb, nev);
+    for (int i = threadIdx.x; i < l * nev; i += blockDim.x) Lb[i] /= w[(unsigned)i % (unsigned)nev];
     __syncthreads();
     // R, L and their products
-    bg<double, double>(nev, (int)N, l, Rb, nev, 1, bs, N, 0, R, N);
-    bg<double, double>(nev, (int)N, l, Lb, nev, 1, bs, N, 0, Lv, N);
-    bg<double, double>(nev, (int)N, l, Rb, nev, 1, bp, N, 0, PR, N);
-    bg<double, double>(nev, (int)N, l, Lb, nev, 1, bm, N, 0, ML, N);
+    EnsProduct ritz[4] = {{nev, (int)N, l, 1, 0, Rb, nev, bs, N, R, N, 1.0, 0.0},
+                          {nev, (int)N, l, 1, 0, Lb, nev, bs, N, Lv, N, 1.0, 0.0},
+                          {nev, (int)N, l, 1, 0, Rb, nev, bp, N, PR, N, 1.0, 0.0},
+                          {nev, (int)N, l, 1, 0, Lb, nev, bm, N, ML, N, 1.0, 0.0}};
+    pg(es, ritz);
     // residuals WL = (A+B)R - w L, WR = (A-B)L - w R
     for (int n = 0; n < nev; ++n) {
       double sL = 0.0, sR = 0.0;
@@ -667,18 +913,19 @@ __device__ void ens_davidson(const EnsMolecule& Mo, double conv, int maxiter, do
     }
     // precondition into bs[l .. l+dk)
     double* Q = bs + (long)l * N;
-    for (long i = threadIdx.x; i < (long)dk * N; i += blockDim.x) {
-      const int t = (int)(i / N);
-      const long e = i - (long)t * N;
+    for (int t = 0; t < dk; ++t) {
       const int src = s_sel[1 + t];
-      const double om = Mo.omega[e];
-      double d = w[src % k] - om;
-      if (fabs(d) < 1.0e-6) d = 1.0e-6 * om;
-      Q[i] = W[(long)src * N + e] / d;
+      const double wt = w[src % k];
+      for (long e = threadIdx.x; e < N; e += blockDim.x) {
+        const double om = Mo.omega[e];
+        double d = wt - om;
+        if (fabs(d) < 1.0e-6) d = 1.0e-6 * om;
+        Q[t * N + e] = W[(long)src * N + e] / d;
+      }
     }
     __syncthreads();
-    const int kept = ens_orthonormalize(bs, l, Q, dk, N, 1.0e-8, (double*)(ws + L.Sq), (double*)(ws + L.G),
-                                        (double*)(ws + L.Lc), (double*)(ws + L.Li), (double*)(ws + L.ref),
+    const int kept = ens_orthonormalize(es, bs, l, Q, dk, N, 1.0e-8, (double*)(ws + L.Sq), (double*)(ws + L.G),
+                                        stg, (double*)(ws + L.Li), (double*)(ws + L.ref),
                                         (double*)(ws + L.Qt), (int*)(ws + L.keep), sh);
     new0 = l;
     l += kept;
@@ -686,7 +933,7 @@ __device__ void ens_davidson(const EnsMolecule& Mo, double conv, int maxiter, do
   // outputs: C = bs Tb, X+Y = R, X-Y = L
   if (code == 1) {
     const int nev = k < l ? k : l;
-    bg<double, double>(nev, (int)N, l, Tb, nev, 1, bs, N, 0, Mo.C, N);
+    pg(es, nev, (int)N, l, Tb, nev, 1, bs, N, 0, Mo.C, N);
     for (long i = threadIdx.x; i < (long)nev * N; i += blockDim.x) {
       Mo.XpY[i] = R[i];
       Mo.XmY[i] = Lv[i];
@@ -697,6 +944,7 @@ __device__ void ens_davidson(const EnsMolecule& Mo, double conv, int maxiter, do
     status[0] = it + 1;
     status[1] = code;
     status[2] = l;
+    __hip_atomic_store(&es.ctl->word, ENS_STARTED | ENS_QUIT, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
 }
@@ -707,20 +955,38 @@ __global__ __launch_bounds__(ENS_THREADS) void ensemble_kernel(const EnsMolecule
   __shared__ double sv[ENS_MAXL];
   __shared__ double sp[ENS_MAXL];
   __shared__ double bnd[2];
-  __shared__ int s_sel[1 + 2 * ENS_MAXK];
+  __shared__ int s_sel[2 + 2 * ENS_MAXK];  // the selection, and the item
   __shared__ double stg[EIG_STAGE_WAVES * EIG_STAGE];
-  const int mi = blockIdx.x;
-  if (mi >= nmol) return;
+  __shared__ double wl[ENS_EIG_LDS * (ENS_EIG_LDS | 1)];
+  const int mi = blockIdx.x % nmol, slot = blockIdx.x / nmol, nb = gridDim.x / nmol;
   const EnsMolecule& Mo = mols[mi];
-  if (Mo.precision == 1)
-    ens_davidson<float>(Mo, conv, maxiter, sh, sv, sp, bnd, s_sel, stg);
+  if (slot > 0) {
+    if (Mo.precision == 1)
+      ens_help<float>(Mo, slot, s_sel);
+    else
+      ens_help<double>(Mo, slot, s_sel);
+  } else if (Mo.precision == 1)
+    ens_davidson<float>(Mo, conv, maxiter, sh, sv, sp, bnd, s_sel, stg, wl, nb);
   else
-    ens_davidson<double>(Mo, conv, maxiter, sh, sv, sp, bnd, s_sel, stg);
+    ens_davidson<double>(Mo, conv, maxiter, sh, sv, sp, bnd, s_sel, stg, wl, nb);
+}
+
+__global__ void ensemble_begin_kernel(const EnsMolecule* __restrict__ mols, int nmol) {
+  const int mi = blockIdx.x * blockDim.x + threadIdx.x;
+  if (mi >= nmol) return;
+  EnsCtl* ctl = (EnsCtl*)((char*)mols[mi].work + ens_layout(mols[mi]).ctl);
+  ctl->word = 0;
+  ctl->done = 0;
 }
 
 extern "C" int dftb_ensemble_solve(const EnsMolecule* mols_dev, int nmol, double conv, int maxiter, void* stream) {
   if (!mols_dev || nmol <= 0 || maxiter <= 0) return DFTB_ERR_ARG;
-  hipLaunchKernelGGL(ensemble_kernel, dim3(nmol), dim3(ENS_THREADS), 0, (hipStream_t)stream, mols_dev, nmol, conv,
+  // leaders come first in the grid; helpers leave a quarter of the chip to other streams
+  int nb = ENS_GRID / nmol;
+  nb = nb < 1 ? 1 : nb > ENS_BLOCKS ? ENS_BLOCKS : nb;
+  hipLaunchKernelGGL(ensemble_begin_kernel, dim3((nmol + 63) / 64), dim3(64), 0, (hipStream_t)stream, mols_dev, nmol);
+  DFTB_CHECK_LAUNCH();
+  hipLaunchKernelGGL(ensemble_kernel, dim3(nmol * nb), dim3(ENS_THREADS), 0, (hipStream_t)stream, mols_dev, nmol, conv,
                      maxiter);
   DFTB_CHECK_LAUNCH();
   return DFTB_OK;
