@@ -28,13 +28,19 @@ struct MvLayout {
 };
 
 // AO exchange intermediates per vector (elements): B1 [2 npad][max(opad, vpad)],
-// BH [2 npad][2 npad], B3 [vpad][2 npad]; BF16x3 keeps two BH (BH and its
-// transpose) and two B3 per vector
+// BH [2 npad][ld], B3 [vpad][ld]; BF16x3 keeps two BH (BH and its transpose) and
+// two B3 per vector.  In BF16x3 the rows of BH and B3 start on 64 bytes (ld % 32 == 0):
+// the GEMMs stage 64-byte row segments, and an unaligned one touches two 64-byte
+// sectors (40 vectors of 672 atoms, 2 npad = 4976: 31.9 ms, now 30.7).
+static long ao_ld(const CasidaOperator* op) {
+  const long np2 = 2L * op->npad;
+  return op->precision == 2 ? (np2 + 31) / 32 * 32 : np2;
+}
 static void ao_sizes(const CasidaOperator* op, long* e1, long* eh, long* e3) {
-  const long np2 = 2L * op->npad, w = op->opad > op->vpad ? op->opad : op->vpad;
+  const long np2 = 2L * op->npad, ld = ao_ld(op), w = op->opad > op->vpad ? op->opad : op->vpad;
   *e1 = np2 * w;
-  *eh = np2 * np2;
-  *e3 = (long)op->vpad * np2;
+  *eh = np2 * ld;
+  *e3 = (long)op->vpad * ld;
 }
 // bytes per element summed over the arrays of one operand (BF16x3: hi + lo)
 static int ao_esz(int precision) { return precision == 0 ? 8 : 4; }
@@ -275,7 +281,7 @@ static int ao_gemm(int prec, const void* A, const void* A2, long lda, const void
 static int ao_exchange(const CasidaOperator* op, const MvLayout& L, char* ws, int nvec, const void* V,
                        const void* Vlo, double* X1, double* X2, hipStream_t st) {
   const int prec = op->precision;
-  const long np2 = 2L * op->npad, opad = op->opad, vpad = op->vpad, N = L.N;
+  const long np2 = 2L * op->npad, ld = ao_ld(op), opad = op->opad, vpad = op->vpad, N = L.N;
   long e1, eh, e3;
   ao_sizes(op, &e1, &eh, &e3);
   const long vs = prec == 0 ? 8 : (prec == 1 ? 4 : 2);   // bytes per vector element (per array)
@@ -307,18 +313,18 @@ static int ao_exchange(const CasidaOperator* op, const MvLayout& L, char* ws, in
       g.out_type = GEMM_OUT_BF16PAIR;
       g.A = op->ao_o[0]; g.A2 = op->ao_o[1]; g.lda = opad; g.sA = 0;
       g.B = b1; g.B2 = b1l; g.ldb = opad; g.sB = e1; g.b_trans = 1;
-      g.C = bh; g.C2 = bhl; g.ldc = np2; g.sC = eh;
-      g.Ct = bh + (size_t)c * eh * es; g.Ct2 = bhl + (size_t)c * eh * es; g.ldct = np2; g.sCt = eh;
+      g.C = bh; g.C2 = bhl; g.ldc = ld; g.sC = eh;
+      g.Ct = bh + (size_t)c * eh * es; g.Ct2 = bhl + (size_t)c * eh * es; g.ldct = ld; g.sCt = eh;
       g.M = (int)np2; g.N = (int)np2; g.K = (int)opad; g.batch = c; g.alpha = 1.0;
       g.had = op->gam_ao; g.hmod = op->npad; g.ldh = op->nat + 1; g.hmap = op->amap;
       g.tile = (op->tile_expand == 256 || op->tile_expand == 512) ? op->tile_expand : 0;
       if ((rc = gemm_launch(g, st))) return rc;
-      if ((rc = ao_gemm(prec, op->ao_cyvt[0], op->ao_cyvt[1], np2, bh, bhl, np2, eh, 1, b3, b3l, np2, e3,
+      if ((rc = ao_gemm(prec, op->ao_cyvt[0], op->ao_cyvt[1], np2, bh, bhl, ld, eh, 1, b3, b3l, ld, e3,
                         (int)vpad, (int)np2, (int)np2, 2 * c, 1.0, false, op, false, st, op->tile_contract))) return rc;
-      if ((rc = ao_gemm(prec, op->ao_w[0], op->ao_w[1], np2, b3, b3l, np2, e3, 1, x1, nullptr, vpad, N, (int)opad,
+      if ((rc = ao_gemm(prec, op->ao_w[0], op->ao_w[1], np2, b3, b3l, ld, e3, 1, x1, nullptr, vpad, N, (int)opad,
                         (int)vpad, (int)np2, c, 0.25, true, op, false, st, op->tile_contract))) return rc;
       const size_t o3 = (size_t)c * e3 * es;
-      if ((rc = ao_gemm(prec, op->ao_w[0], op->ao_w[1], np2, b3 + o3, b3l + o3, np2, e3, 1, x2, nullptr, vpad, N,
+      if ((rc = ao_gemm(prec, op->ao_w[0], op->ao_w[1], np2, b3 + o3, b3l + o3, ld, e3, 1, x2, nullptr, vpad, N,
                         (int)opad, (int)vpad, (int)np2, c, 0.25, true, op, false, st, op->tile_contract))) return rc;
       continue;
     }
@@ -406,9 +412,11 @@ extern "C" int dftb_casida_matvec(const CasidaOperator* op, const double* V, int
   if (op->lc) {
     double* X1 = (double*)(ws + L.x1);
     double* X2 = (double*)(ws + L.x2);
-    hipLaunchKernelGGL(zero_kernel, sgrid(total), dim3(256), 0, st, X1, total);
-    hipLaunchKernelGGL(zero_kernel, sgrid(total), dim3(256), 0, st, X2, total);
-    DFTB_CHECK_LAUNCH();
+    if (op->exchange != 1) {   // (the AO exchange writes every entry)
+      hipLaunchKernelGGL(zero_kernel, sgrid(total), dim3(256), 0, st, X1, total);
+      hipLaunchKernelGGL(zero_kernel, sgrid(total), dim3(256), 0, st, X2, total);
+      DFTB_CHECK_LAUNCH();
+    }
     const int it = prec == 0 ? GEMM_IN_F64 : (prec == 1 ? GEMM_IN_F32 : GEMM_IN_BF16X3);
     const int ot = prec == 0 ? GEMM_OUT_F64 : (prec == 1 ? GEMM_OUT_F32 : GEMM_OUT_BF16PAIR);
     const long opad = op->opad, vpad = op->vpad, nat = op->nat;
