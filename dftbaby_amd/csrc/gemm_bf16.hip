@@ -682,14 +682,34 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf3_pipe_kernel(GemmArgs p) {
 #define DFTB_BF3_WAVES 8
 #endif
 
+// Tile rule (all tiles add the same products in the same order): the least of three estimates in
+// us.  The pipelined kernel takes one round per 256 tiles, 1.25 us per 32 k with 256 x 128 tiles
+// and 1.95 (half the chip) to 2.2 us with 256 x 256 ones, plus the epilogue; 64 x 64 tiles share
+// their CU, at 0.7 us per 32 k until about 500 of them and 1.5 ns per tile beyond.  Measured, us
+// (256 x 256, 256 x 128, 64 x 64): 1248 x 1248 x 4976 299, 184, 127; twice that 297, 185, 215;
+// eight times 337, 399, 740; 4976 x 1248 x 1248 92, 63, 100; 176 x 176 x 744 53, 32, 18.
+static int bf3_tile(const GemmArgs& p) {
+  const double stages = ceil_div(p.kchunk < p.K ? p.kchunk : p.K, P_BK), z = (double)p.batch * p.ksplit;
+  const double rows = ceil_div(p.M, P_BM) * z;
+  const double n512 = rows * ceil_div(p.N, 256), n256 = rows * ceil_div(p.N, 128);
+  const double n64 = (double)ceil_div(p.M, 64) * ceil_div(p.N, 64) * z;
+  const double r512 = ceil(n512 / 256), r256 = ceil(n256 / 256);
+  // the transposed copy's epilogue costs about four times the plain one
+  const double t512 = r512 * (stages * (n512 > 128 ? 2.2 : 1.95) + (p.Ct ? 60.0 : 15.0));
+  const double t256 = r256 * (stages * 1.25 + (p.Ct ? 33.0 : 12.0));
+  const double t64 = stages * ((n64 > 467 ? 0.0015 * n64 : 0.7) + 0.12) + 5.0;
+  if (!p.Ct && t64 < t512 && t64 < t256) return 64;
+  return t256 < t512 ? 256 : 512;
+}
+
 int gemm_bf16x3_launch(const GemmArgs& p, hipStream_t st) {
   if (p.a_trans || !p.b_trans) return DFTB_ERR_ARG;
   if (!p.A2 || !p.B2) return DFTB_ERR_ARG;
   if ((p.lda & 7) || (p.ldb & 7) || (p.K & 7) || (p.sA & 7) || (p.sB & 7)) return DFTB_ERR_ARG;
   if (p.ksplit > 1 && (p.kchunk & 7)) return DFTB_ERR_ARG;
   if ((((uintptr_t)p.A) | ((uintptr_t)p.A2) | ((uintptr_t)p.B) | ((uintptr_t)p.B2)) & 15) return DFTB_ERR_ARG;
-  const bool small = p.tile == 64 || (p.tile == 0 && (p.M < 128 || p.N < 128));
-  bool pipe = p.tile == 256 || p.tile == 512 || (p.tile == 0 && p.M >= 256 && p.N >= 128 && p.K >= 4 * P_BK);
+  const int tile = p.tile ? p.tile : bf3_tile(p);
+  bool pipe = tile == 256 || tile == 512;
   if (p.Ct) {
     // transposed copy: pipelined kernel, 16x16 form, bf16 pairs stored as 16-byte
     // row segments (8 rows), so M, ldct, sCt multiples of 8 and 16-byte aligned arrays
@@ -699,10 +719,10 @@ int gemm_bf16x3_launch(const GemmArgs& p, hipStream_t st) {
     pipe = true;
   }
   if (pipe) {
-    // tile 256: 256 x 128 tiles; tile 512: 256 x 256 tiles; automatic: 256 x 256
-    // when N >= 256 unless DFTB_BF3_BN=128 asks for the narrower tile
+    // tile 256: 256 x 128 tiles; tile 512: 256 x 256 tiles, unless DFTB_BF3_BN=128 asks for
+    // the narrower one where the rule chose it
     static const int bn_env = getenv("DFTB_BF3_BN") ? atoi(getenv("DFTB_BF3_BN")) : 256;
-    const int bn = p.tile == 512 ? 256 : p.tile == 256 ? 128 : (bn_env == 128 || p.N < 256) ? 128 : 256;
+    const int bn = tile != 512 || (p.tile == 0 && bn_env == 128) ? 128 : 256;
     // 32-bit buffer offsets: each workgroup's operand span must stay below 4 GiB
     const long span_a = ((long)P_BM * p.lda + p.K) * 2, span_b = ((long)bn * p.ldb + p.K) * 2;
     if (span_a >= 0xffff0000L || span_b >= 0xffff0000L) return DFTB_ERR_ARG;
@@ -737,7 +757,7 @@ int gemm_bf16x3_launch(const GemmArgs& p, hipStream_t st) {
   }
   GemmTimer tm;
   tm.begin(st);
-  if (small) {
+  if (tile == 64) {
     dim3 grid(ceil_div(p.N, 64), ceil_div(p.M, 64), p.batch * p.ksplit);
     hipLaunchKernelGGL((gemm_bf3_kernel<64, 64>), grid, dim3(256), 0, st, p);
   } else {

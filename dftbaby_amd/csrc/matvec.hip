@@ -321,11 +321,14 @@ static int ao_exchange(const CasidaOperator* op, const MvLayout& L, char* ws, in
       if ((rc = gemm_launch(g, st))) return rc;
       if ((rc = ao_gemm(prec, op->ao_cyvt[0], op->ao_cyvt[1], np2, bh, bhl, ld, eh, 1, b3, b3l, ld, e3,
                         (int)vpad, (int)np2, (int)np2, 2 * c, 1.0, false, op, false, st, op->tile_contract))) return rc;
+      // one launch for both where X2 follows X1 (all vectors at once)
+      const bool both = x2 == x1 + (size_t)c * N;
       if ((rc = ao_gemm(prec, op->ao_w[0], op->ao_w[1], np2, b3, b3l, ld, e3, 1, x1, nullptr, vpad, N, (int)opad,
-                        (int)vpad, (int)np2, c, 0.25, true, op, false, st, op->tile_contract))) return rc;
+                        (int)vpad, (int)np2, both ? 2 * c : c, 0.25, true, op, false, st, op->tile_contract))) return rc;
       const size_t o3 = (size_t)c * e3 * es;
-      if ((rc = ao_gemm(prec, op->ao_w[0], op->ao_w[1], np2, b3 + o3, b3l + o3, ld, e3, 1, x2, nullptr, vpad, N,
-                        (int)opad, (int)vpad, (int)np2, c, 0.25, true, op, false, st, op->tile_contract))) return rc;
+      if (!both && (rc = ao_gemm(prec, op->ao_w[0], op->ao_w[1], np2, b3 + o3, b3l + o3, ld, e3, 1, x2, nullptr, vpad,
+                                 N, (int)opad, (int)vpad, (int)np2, c, 0.25, true, op, false, st,
+                                 op->tile_contract))) return rc;
       continue;
     }
     if ((rc = ao_gemm(prec, op->ao_o[0], op->ao_o[1], opad, b1, b1l, opad, e1, 1, bh, bhl, np2, eh, (int)np2,
