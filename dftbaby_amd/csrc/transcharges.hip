@@ -76,6 +76,83 @@ __global__ __launch_bounds__(256) void tc_kernel(const double* __restrict__ Xp, 
   }
 }
 
+// Contiguous output rows that are no multiple of a 128-byte line (the reference layout with an odd
+// block): the same products, but whole rows go to LDS first, R at a time and two buffers, and
+// leave as 16-byte stores of whole lines, so that only a chunk's first and last line are written
+// in parts (non-temporal: 6% faster).  q runs over S * 256 >= Q, one q per thread and stripe.  Bound by the HBM writes:
+// q_oo, q_ov and q_vv of 501 atoms, 927 x 921 orbitals (10.3 GB) take 1.97 ms, by tc_kernel 2.45.
+// Dynamic LDS: 2 (R Q + 16) doubles, then the 2 NMU pchunk doubles of the p rows.
+typedef double tc_d2 __attribute__((ext_vector_type(2)));
+template <int NMU, int S>
+__global__ __launch_bounds__(256) void tc_flat_kernel(const double* __restrict__ Xp, const double* __restrict__ Yp,
+                                                      int P, const double* __restrict__ Xq,
+                                                      const double* __restrict__ Yq, int Q,
+                                                      const int* __restrict__ atom_off, int pchunk, int R,
+                                                      double* __restrict__ out) {
+  extern __shared__ __attribute__((aligned(16))) double lds[];
+  const int A = blockIdx.x;
+  const int pbeg = blockIdx.y * pchunk, pend = min(P, pbeg + pchunk);
+  const int mu0 = atom_off[A];
+  const int nmu = atom_off[A + 1] - mu0;
+  const int bsz = (R * Q + 16 + 1) & ~1;
+  double* sxy = lds + 2 * bsz;           // [pchunk][NMU][2]
+  for (int t = threadIdx.x; t < (pend - pbeg) * NMU; t += blockDim.x) {
+    const int pp = t / NMU, mu = t % NMU;
+    const bool ok = mu < nmu;
+    const long idx = ok ? (long)(mu0 + mu) * P + pbeg + pp : 0;
+    const double x = Xp[idx], y = Yp[idx];
+    sxy[2 * t] = ok ? x : 0.0;
+    sxy[2 * t + 1] = ok ? y : 0.0;
+  }
+  double xq[S][NMU], yq[S][NMU];
+#pragma unroll
+  for (int j = 0; j < S; ++j) {
+    const int q = threadIdx.x + 256 * j;
+#pragma unroll
+    for (int mu = 0; mu < NMU; ++mu) {
+      const bool ok = (q < Q) && (mu < nmu);
+      const long idx = ok ? (long)(mu0 + mu) * Q + q : 0;
+      const double x = Xq[idx], y = Yq[idx];
+      xq[j][mu] = ok ? x : 0.0;
+      yq[j][mu] = ok ? y : 0.0;
+    }
+  }
+  __syncthreads();
+  const double* r = sxy;
+  int cur = 0;
+  for (int p0 = pbeg; p0 < pend; p0 += R, cur ^= 1) {
+    const int nr = min(R, pend - p0);
+    double* o = out + ((long)A * P + p0) * Q;
+    const int ph = (int)(((uintptr_t)o >> 3) & 15);   // place of the first result in its line
+    double* buf = lds + cur * bsz;
+    double* b = buf + ph + threadIdx.x;
+    for (int p = 0; p < nr; ++p, r += 2 * NMU, b += Q) {
+      double rv[2 * NMU];
+#pragma unroll
+      for (int i = 0; i < 2 * NMU; ++i) rv[i] = r[i];
+#pragma unroll
+      for (int j = 0; j < S; ++j) {
+        double s = 0.0;
+#pragma unroll
+        for (int mu = 0; mu < NMU; ++mu) s += rv[2 * mu] * yq[j][mu] + xq[j][mu] * rv[2 * mu + 1];
+        if ((int)threadIdx.x + 256 * j < Q) b[256 * j] = 0.5 * s;
+      }
+    }
+    // the other buffer's reads lie behind this barrier, two steps before its next writes
+    __syncthreads();
+    const int end = ph + nr * Q;
+    double* line = o - ph;
+    for (int i = 2 * threadIdx.x; i < end; i += 512) {
+      if (i >= ph && i + 1 < end) {
+        __builtin_nontemporal_store(*(const tc_d2*)(buf + i), (tc_d2*)(line + i));
+      } else {
+        if (i >= ph) line[i] = buf[i];
+        if (i + 1 >= ph && i + 1 < end) line[i + 1] = buf[i + 1];
+      }
+    }
+  }
+}
+
 template <int NMU, int S>
 static void tc_launch(dim3 grid, size_t lds, hipStream_t st, const double* Xp, const double* Yp, int P,
                       const double* Xq, const double* Yq, int Q, const int* off, int Ppad, int Qpad, int pchunk,
@@ -91,6 +168,22 @@ static void tc_dispatch(int S, dim3 grid, size_t lds, hipStream_t st, const doub
                         double* out, long sP, long sA) {
 #define TC_CASE(n) \
   case n: tc_launch<NMU, (NMU * n <= 32 ? n : 1)>(grid, lds, st, Xp, Yp, P, Xq, Yq, Q, off, Ppad, Qpad, pchunk, out, sP, sA); break;
+  switch (S) {
+    TC_CASE(1) TC_CASE(2) TC_CASE(3) TC_CASE(4) TC_CASE(5) TC_CASE(6) TC_CASE(7) TC_CASE(8)
+    default: break;
+  }
+#undef TC_CASE
+}
+
+template <int NMU>
+static void tc_flat_dispatch(int S, dim3 grid, size_t lds, hipStream_t st, const double* Xp, const double* Yp, int P,
+                             const double* Xq, const double* Yq, int Q, const int* off, int pchunk, int R,
+                             double* out) {
+#define TC_CASE(n)                                                                                             \
+  case n:                                                                                                      \
+    hipLaunchKernelGGL((tc_flat_kernel<NMU, (NMU * n <= 32 ? n : 1)>), grid, dim3(256), lds, st, Xp, Yp, P, Xq, Yq, \
+                       Q, off, pchunk, R, out);                                                                \
+    break;
   switch (S) {
     TC_CASE(1) TC_CASE(2) TC_CASE(3) TC_CASE(4) TC_CASE(5) TC_CASE(6) TC_CASE(7) TC_CASE(8)
     default: break;
@@ -120,10 +213,26 @@ static int tc_block(const TcPlan& t, bool p_occ, bool q_occ, int Ppad, int Qpad,
   const int stripes = ceil_div(Qpad, 256);
   const int S = stripes < smax ? stripes : smax;
   const int gz = ceil_div(stripes, S);
-  // p chunks: output rows that are not 128-byte aligned (the reference layout
-  // with nocc or nvirt not a multiple of 16) leave partial lines at row ends,
-  // merged best by short chunks (16 rows: 4.8 TB/s against 3.5 TB/s with 624 at
-  // the flake); aligned rows stream best in long chunks (>= ~1024 workgroups)
+  // contiguous rows that are not aligned to lines
+  if (Qpad == Q && Ppad == P && sP == Q && sA == (long)P * Q && gz == 1 && ((Q % 16) != 0 || ((uintptr_t)out & 127))) {
+    // 16 KB per buffer and 32 rows: of 1024 .. 8192 doubles and 16 .. 128 rows the best
+    // or within 2% of it (501 and 300 atoms)
+    const int R = Q < 1024 ? 2048 / Q : 1, pchunk = P < 32 ? P : 32;
+    const size_t lds = ((size_t)2 * ((R * Q + 17) & ~1) + (size_t)2 * nmu * pchunk) * sizeof(double);
+    dim3 grid(t.nat, ceil_div(P, pchunk));
+    if (nmu == 4)
+      tc_flat_dispatch<4>(S, grid, lds, st, Xp, Yp, P, Xq, Yq, Q, t.off, pchunk, R, out);
+    else if (nmu == 9)
+      tc_flat_dispatch<9>(S, grid, lds, st, Xp, Yp, P, Xq, Yq, Q, t.off, pchunk, R, out);
+    else
+      tc_flat_dispatch<16>(S, grid, lds, st, Xp, Yp, P, Xq, Yq, Q, t.off, pchunk, R, out);
+    DFTB_CHECK_LAUNCH();
+    return DFTB_OK;
+  }
+  // p chunks: rows too long for tc_flat_kernel that are not 128-byte aligned leave
+  // partial lines at row ends, merged best by short chunks (16 rows: 4.8 TB/s against
+  // 3.5 TB/s with 624 at the flake); aligned rows stream best in long chunks (>= ~1024
+  // workgroups)
   const int pmax = (int)(TC_LDS_BYTES / (2 * nmu * sizeof(double)));
   int pchunk;
   if ((sP % 16) != 0 || (sA % 16) != 0) {
