@@ -168,12 +168,12 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmArgs p) {
     }
 }
 
-// Sum split-K partials: C[b][i] = alpha * sum_s P[s][b][i] + beta * C[b][i]  (dense, row-major M x N)
+// Sum split-K partials: C[b][i] = alpha * sum_s P[s][b][i] + beta * C[b][i]  (dense, row-major M x N).
+// One wave per workgroup: few entries and many slices leave few waves, which then spread over CUs.
 __global__ void gemm_reduce_kernel(const double* P, long sP, int nsplit, double* C, long n, double alpha, double beta) {
   long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  double s = 0.0;
-  for (int k = 0; k < nsplit; ++k) s += P[k * sP + i];
+  double s = sum_slices(P + i, sP, nsplit);
   s *= alpha;
   if (beta != 0.0) s += beta * C[i];
   C[i] = s;
@@ -294,7 +294,7 @@ int gemm_launch(const GemmArgs& p0, hipStream_t st, bool timed) {
 
 int gemm_reduce_launch(const double* P, long sP, int nsplit, double* C, long n, double alpha, double beta, hipStream_t st) {
   if (n <= 0) return DFTB_OK;
-  hipLaunchKernelGGL(gemm_reduce_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, st, P, sP, nsplit, C, n, alpha, beta);
+  hipLaunchKernelGGL(gemm_reduce_kernel, dim3(ceil_div(n, 64)), dim3(64), 0, st, P, sP, nsplit, C, n, alpha, beta);
   DFTB_CHECK_LAUNCH();
   return DFTB_OK;
 }
