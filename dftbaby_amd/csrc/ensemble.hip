@@ -320,18 +320,31 @@ struct EnsCtl {
   char pad0[120];
   unsigned long long done;                 // items finished by helpers since the launch began
   char pad1[120];
+  unsigned long long here;                 // helpers that have started
+  char pad2[120];
   EnsTask task;
 };
 
 struct EnsShare {                          // the leader's view
   EnsCtl* ctl;
-  int nb;                                  // blocks of this molecule
+  int nb;                                  // blocks at work on this molecule when last counted
+  int cap;                                 // most of them
   int* s_item;                             // LDS
   unsigned long long done;                 // items that helpers have finished so far
 };
 
 __device__ __forceinline__ unsigned long long ens_load(const unsigned long long* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Counts the helpers: where none run (other work holds the CUs), products stay in one piece.
+__device__ __forceinline__ void ens_count(EnsShare& sh) {
+  if (sh.nb >= sh.cap) return;
+  if (threadIdx.x == 0) *sh.s_item = (int)ens_load(&sh.ctl->here);
+  __syncthreads();
+  const int nb = 1 + *sh.s_item;
+  __syncthreads();
+  sh.nb = nb < sh.cap ? nb : sh.cap;
 }
 
 // next item of the current section, or -1.  One thread's fences and the barriers around them
@@ -575,12 +588,17 @@ __device__ void ens_help(const EnsMolecule& Mo, int slot, int* s_item) {
   if (slot >= L.slots) return;
   const unsigned long long mask = (1ull << ENS_ITEM_BITS) - 1;
   const unsigned long long t0 = wall_clock64();
+  bool counted = false;
   for (;;) {
     if (threadIdx.x == 0) {
       // -1: the leader has ended, or did not start within 0.2 ms (100 MHz clock); 1: an item may be free
       int go = 0;
       while (!go) {
         const unsigned long long w = ens_load(&ctl->word);
+        if ((w & ENS_STARTED) && !counted) {
+          __hip_atomic_fetch_add(&ctl->here, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          counted = true;
+        }
         if ((w & ENS_QUIT) || (!(w & ENS_STARTED) && wall_clock64() - t0 > 20000))
           go = -1;
         else if ((w & mask) < ((w >> ENS_ITEM_BITS) & mask))
@@ -742,7 +760,7 @@ __device__ void ens_davidson(const EnsMolecule& Mo, double conv, int maxiter, do
                              double* bnd, int* s_sel, double* stg, double* wl, int nb) {
   char* ws = (char*)Mo.work;
   const EnsLayout L = ens_layout(Mo);
-  EnsShare es = {(EnsCtl*)(ws + L.ctl), nb < L.slots ? nb : L.slots, s_sel + 2 * ENS_MAXK + 1, 0};
+  EnsShare es = {(EnsCtl*)(ws + L.ctl), 1, nb < L.slots ? nb : L.slots, s_sel + 2 * ENS_MAXK + 1, 0};
   if (threadIdx.x == 0)
     __hip_atomic_store(&es.ctl->word, ENS_STARTED, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
   const long N = (long)Mo.opad * Mo.vpad;
@@ -778,6 +796,7 @@ __device__ void ens_davidson(const EnsMolecule& Mo, double conv, int maxiter, do
   int code = 0, it = 0;
   for (it = 0; it < maxiter; ++it) {
     const int m = l - new0;
+    ens_count(es);
     if (m > 0) {
       ens_matvec<T>(es, Mo, ws, L, bs + (long)new0 * N, m, bp + (long)new0 * N, bm + (long)new0 * N);
       // new columns/rows of M+- = bs^T (A+-B) bs
@@ -808,6 +827,7 @@ __device__ void ens_davidson(const EnsMolecule& Mo, double conv, int maxiter, do
       }
       __syncthreads();
     }
+    ens_count(es);
     // subspace step (Solver.py:759-798)
     if (ens_sqrtm(es, Mm, l, cap, Sq, Sinv, (double*)(ws + L.Tns), (double*)(ws + L.P), (double*)(ws + L.Y2),
                   (double*)(ws + L.Z2), sh)) {
@@ -977,12 +997,15 @@ __global__ void ensemble_begin_kernel(const EnsMolecule* __restrict__ mols, int 
   EnsCtl* ctl = (EnsCtl*)((char*)mols[mi].work + ens_layout(mols[mi]).ctl);
   ctl->word = 0;
   ctl->done = 0;
+  ctl->here = 0;
 }
 
 extern "C" int dftb_ensemble_solve(const EnsMolecule* mols_dev, int nmol, double conv, int maxiter, void* stream) {
   if (!mols_dev || nmol <= 0 || maxiter <= 0) return DFTB_ERR_ARG;
-  // leaders come first in the grid; helpers leave a quarter of the chip to other streams
-  int nb = ENS_GRID / nmol;
+  // leaders come first in the grid; helpers leave a quarter of the chip to other streams.  From
+  // ENS_GRID molecules on the leaders take the chip anyway, and helpers start as members end
+  // (256 polyenes C8-C40: 2.25 s without helpers, 1.18 so).
+  int nb = nmol >= ENS_GRID ? ENS_BLOCKS : ENS_GRID / nmol;
   nb = nb < 1 ? 1 : nb > ENS_BLOCKS ? ENS_BLOCKS : nb;
   hipLaunchKernelGGL(ensemble_begin_kernel, dim3((nmol + 63) / 64), dim3(64), 0, (hipStream_t)stream, mols_dev, nmol);
   DFTB_CHECK_LAUNCH();

@@ -287,9 +287,9 @@ int dftb_unit_vectors(const long* idx, int k, long n, double* X, void* stream);
 /* ---- batched ensemble: one persistent launch ---------------------------------
  * Solves the lowest k roots of the non-Hermitian Casida problem (the algorithm
  * of Solver.py:637-917) for many molecules of uneven size in one launch: one
- * workgroup per molecule runs its whole Davidson loop on the device; in launches
- * of up to 96 molecules further workgroups (up to 7 each, 192 in all) take part of
- * its products, with the same results.  The host
+ * workgroup per molecule runs its whole Davidson loop on the device; further
+ * workgroups (up to 7 each, 192 in all while there are fewer molecules than that)
+ * take part of its products, with the same results.  The host
  * fills one EnsMolecule per molecule (device array, largest first): charges in
  * the engine layouts (FP64, plus FP32 copies q32 = {q_oo, q_ov, qf_ov, qf_vv}
  * for precision 1), nguess initial unit-vector indices, the expansion storage
