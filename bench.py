@@ -512,7 +512,7 @@ def run_ensemble(args, log):
     t_launch = float(np.mean(t_solve))
     roof = {"bound": "mfma", "achieved": flops / t_launch / 1e12, "peak": PEAK["fp32"] / 1e12, "unit": "TFLOP/s",
             "frac": flops / t_launch / PEAK["fp32"], "traffic": None,
-            "kernel": "ensemble_kernel (one workgroup per molecule; FP32 exchange products)",
+            "kernel": "ensemble_kernel (one leading workgroup per molecule; FP32 exchange products)",
             "vectors": int(sum(res.vectors))}
     cpu = None
     if not args.no_cpu_baseline:
