@@ -798,9 +798,9 @@ def main():
     if B["prec"] == "bf16x3":
         cls, kname, peak = "bf16x3_pipe", "gemm_bf3_pipe_kernel<8>", PEAK["bf16x3"]
     elif B["prec"] == "fp32":
-        cls, kname, peak = "f32_128", "gemm_fp_kernel<float, 128, 128, 32, false, false>", PEAK["fp32"]
+        cls, kname, peak = "f32_128", "gemm_f32_kernel<128, 128, 32, false, false>", PEAK["fp32"]
     else:
-        cls, kname, peak = "f64_128", "gemm_fp_kernel<double, 128, 128, 16, false, false>", PEAK["fp64"]
+        cls, kname, peak = "f64_128", "gemm_f64_kernel<4, 4, 2, 2, 1, false, false>", PEAK["fp64"]
     sec, n, fl = B["kern"].get(cls, (0.0, 0, 0.0))
     achieved = fl / sec if sec > 0 else 0.0
     tr = traffic_per_launch(kname, args.workload, B["exchange"])
