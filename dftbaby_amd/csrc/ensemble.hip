@@ -337,6 +337,29 @@ __device__ __forceinline__ unsigned long long ens_load(const unsigned long long*
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Every wave's stores have reached the L2 before the block goes on.  A barrier alone waits for LDS
+// (within a CU stores stay in order), and a release by one thread for the stores of its own wave:
+// another wave's could still be on their way when that thread writes the L2 back, and a block on
+// another XCD would read what was there before.
+__device__ __forceinline__ void ens_stores_done() {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+}
+
+// One thread, after ens_stores_done(): the L2 is written back, and that has ended, before the word
+// that hands the stores over.
+__device__ __forceinline__ void ens_release() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// One thread, after reading such a word and before a barrier: L1 and L2 have dropped what is
+// stale when the block's other waves read.
+__device__ __forceinline__ void ens_acquire() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 // Counts the helpers: where none run (other work holds the CUs), products stay in one piece.
 __device__ __forceinline__ void ens_count(EnsShare& sh) {
   if (sh.nb >= sh.cap) return;
@@ -347,8 +370,7 @@ __device__ __forceinline__ void ens_count(EnsShare& sh) {
   sh.nb = nb < sh.cap ? nb : sh.cap;
 }
 
-// next item of the current section, or -1.  One thread's fences and the barriers around them
-// order the accesses of the whole block.
+// next item of the current section, or -1
 template <bool HELPER>
 __device__ __forceinline__ int ens_take(EnsCtl* ctl, int* s_item) {
   if (threadIdx.x == 0) {
@@ -356,7 +378,7 @@ __device__ __forceinline__ int ens_take(EnsCtl* ctl, int* s_item) {
         __hip_atomic_fetch_add(&ctl->word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const unsigned long long mask = (1ull << ENS_ITEM_BITS) - 1, idx = old & mask;
     *s_item = (old & ENS_QUIT) || idx >= ((old >> ENS_ITEM_BITS) & mask) ? -1 : (int)idx;
-    if (HELPER) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (HELPER) ens_acquire();
   }
   __syncthreads();
   const int item = *s_item;
@@ -367,10 +389,12 @@ __device__ __forceinline__ int ens_take(EnsCtl* ctl, int* s_item) {
 template <typename F>
 __device__ __forceinline__ void ens_section(EnsShare& sh, int items, F&& run) {
   // thread 0 has written the task
-  __syncthreads();
-  if (threadIdx.x == 0)
-    __hip_atomic_store(&sh.ctl->word, ENS_STARTED | ((unsigned long long)items << ENS_ITEM_BITS), __ATOMIC_RELEASE,
+  ens_stores_done();
+  if (threadIdx.x == 0) {
+    ens_release();
+    __hip_atomic_store(&sh.ctl->word, ENS_STARTED | ((unsigned long long)items << ENS_ITEM_BITS), __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
+  }
   int mine = 0;
   for (int i = ens_take<false>(sh.ctl, sh.s_item); i >= 0; i = ens_take<false>(sh.ctl, sh.s_item)) {
     run(i);
@@ -379,7 +403,7 @@ __device__ __forceinline__ void ens_section(EnsShare& sh, int items, F&& run) {
   sh.done += items - mine;
   if (threadIdx.x == 0) {
     while (ens_load(&sh.ctl->done) != sh.done) __builtin_amdgcn_s_sleep(1);
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    ens_acquire();
   }
   __syncthreads();
 }
@@ -619,8 +643,11 @@ __device__ void ens_help(const EnsMolecule& Mo, int slot, int* s_item) {
       ens_exchange<T>(Mo, ws, L, slot, t->V, i, t->outP, t->outM);
     else
       ens_product_item(t, i);
-    __syncthreads();
-    if (threadIdx.x == 0) __hip_atomic_fetch_add(&ctl->done, 1ull, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    ens_stores_done();
+    if (threadIdx.x == 0) {
+      ens_release();
+      __hip_atomic_fetch_add(&ctl->done, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
   }
 }
 
@@ -762,7 +789,7 @@ __device__ void ens_davidson(const EnsMolecule& Mo, double conv, int maxiter, do
   const EnsLayout L = ens_layout(Mo);
   EnsShare es = {(EnsCtl*)(ws + L.ctl), 1, nb < L.slots ? nb : L.slots, s_sel + 2 * ENS_MAXK + 1, 0};
   if (threadIdx.x == 0)
-    __hip_atomic_store(&es.ctl->word, ENS_STARTED, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&es.ctl->word, ENS_STARTED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // hands nothing over
   const long N = (long)Mo.opad * Mo.vpad;
   const int k = Mo.k, cap = Mo.cap;
   const long kmax = (long)Mo.nocc * Mo.nvirt;
@@ -964,7 +991,7 @@ __device__ void ens_davidson(const EnsMolecule& Mo, double conv, int maxiter, do
     status[0] = it + 1;
     status[1] = code;
     status[2] = l;
-    __hip_atomic_store(&es.ctl->word, ENS_STARTED | ENS_QUIT, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&es.ctl->word, ENS_STARTED | ENS_QUIT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
 }
