@@ -682,12 +682,19 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf3_pipe_kernel(GemmArgs p) {
 #define DFTB_BF3_WAVES 8
 #endif
 
+// the pipelined kernel addresses the rows of a tile by 32-bit offsets
+static bool bf3_span_ok(const GemmArgs& p, int bn) {
+  const long span_a = ((long)P_BM * p.lda + p.K) * 2, span_b = ((long)bn * p.ldb + p.K) * 2;
+  return span_a < 0xffff0000L && span_b < 0xffff0000L;
+}
+
 // Tile rule (all tiles add the same products in the same order): the least of three estimates in
 // us.  The pipelined kernel takes one round per 256 tiles, 1.25 us per 32 k with 256 x 128 tiles
 // and 1.95 (half the chip) to 2.2 us with 256 x 256 ones, plus the epilogue; 64 x 64 tiles share
 // their CU, at 0.7 us per 32 k until about 500 of them and 1.5 ns per tile beyond.  Measured, us
 // (256 x 256, 256 x 128, 64 x 64): 1248 x 1248 x 4976 299, 184, 127; twice that 297, 185, 215;
 // eight times 337, 399, 740; 4976 x 1248 x 1248 92, 63, 100; 176 x 176 x 744 53, 32, 18.
+// Rows too long for a pipelined tile's offsets go to the narrower one or to 64 x 64 tiles.
 static int bf3_tile(const GemmArgs& p) {
   const double stages = ceil_div(p.kchunk < p.K ? p.kchunk : p.K, P_BK), z = (double)p.batch * p.ksplit;
   const double rows = ceil_div(p.M, P_BM) * z;
@@ -698,8 +705,9 @@ static int bf3_tile(const GemmArgs& p) {
   const double t512 = r512 * (stages * (n512 > 128 ? 2.2 : 1.95) + (p.Ct ? 60.0 : 15.0));
   const double t256 = r256 * (stages * 1.25 + (p.Ct ? 33.0 : 12.0));
   const double t64 = stages * ((n64 > 467 ? 0.0015 * n64 : 0.7) + 0.12) + 5.0;
-  if (!p.Ct && t64 < t512 && t64 < t256) return 64;
-  return t256 < t512 ? 256 : 512;
+  const bool ok512 = bf3_span_ok(p, 256), ok256 = bf3_span_ok(p, 128);
+  if (!p.Ct && (!ok256 || (t64 < t512 && t64 < t256))) return 64;
+  return !ok512 || t256 < t512 ? 256 : 512;
 }
 
 int gemm_bf16x3_launch(const GemmArgs& p, hipStream_t st) {
@@ -723,9 +731,7 @@ int gemm_bf16x3_launch(const GemmArgs& p, hipStream_t st) {
     // the narrower one where the rule chose it
     static const int bn_env = getenv("DFTB_BF3_BN") ? atoi(getenv("DFTB_BF3_BN")) : 256;
     const int bn = tile != 512 || (p.tile == 0 && bn_env == 128) ? 128 : 256;
-    // 32-bit buffer offsets: each workgroup's operand span must stay below 4 GiB
-    const long span_a = ((long)P_BM * p.lda + p.K) * 2, span_b = ((long)bn * p.ldb + p.K) * 2;
-    if (span_a >= 0xffff0000L || span_b >= 0xffff0000L) return DFTB_ERR_ARG;
+    if (!bf3_span_ok(p, bn)) return DFTB_ERR_ARG;
     dim3 grid(ceil_div(p.N, bn), ceil_div(p.M, P_BM), p.batch * p.ksplit);
     GemmTimer tm;
     tm.begin(st);
