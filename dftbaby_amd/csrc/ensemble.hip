@@ -500,7 +500,7 @@ __host__ __device__ static EnsLayout ens_layout(const EnsMolecule& m) {
   const long cap = m.cap, k = m.k;
   // one TT per block while they stay within 256 MB
   L.tt = al256((size_t)m.nat * rows * m.vpad * 8);
-  const size_t fit = ((size_t)1 << 28) / L.tt;
+  const size_t fit = L.tt > 0 ? ((size_t)1 << 28) / L.tt : 1;
   L.slots = fit < 1 ? 1 : fit > ENS_BLOCKS ? ENS_BLOCKS : (int)fit;
   size_t o = 0;
   size_t* fields[] = {&L.TT, &L.X1, &L.X2, &L.tv, &L.gv, &L.Sq, &L.Sinv, &L.H, &L.Y2, &L.Z2, &L.P, &L.Tns, &L.eig,

@@ -90,3 +90,18 @@ def test_noalloc_trans_charges_rejects_sizes_beyond_its_scratch():
         _lib.DFTB_ERR_ARG
     assert lib.dftb_trans_charges_noalloc(fake, fake, fake, opa, 1, 4, -1, 2, fake, fake, fake, None) == \
         _lib.DFTB_ERR_ARG
+
+
+@pytest.mark.parametrize("empty", ["nat", "vpad", "opad"])
+def test_ensemble_workspace_of_an_empty_molecule(empty):
+    """A molecule without atoms, virtual or occupied orbitals has a size too (in a process of its
+    own: a division by its empty expansion buffer ends the program)."""
+    import subprocess
+    import sys
+    from dftbaby_amd import _lib
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("HIP library not built")
+    code = ("import ctypes\nfrom dftbaby_amd import _lib\nm = _lib.EnsMolecule()\n"
+            "m.nat = m.nocc = m.nvirt = m.opad = m.vpad = m.k = m.cap = m.nguess = 8\n"
+            "m.%s = 0\nassert _lib.load().dftb_ensemble_workspace(ctypes.byref(m)) > 0\n" % empty)
+    assert subprocess.run([sys.executable, "-c", code], cwd=ROOT).returncode == 0
