@@ -113,6 +113,7 @@ _SIGS = {
     "dftb_symmetrize": (_i, [_vp, _i, _i, _vp, _vp]),
     "dftb_coldot": (_i, [_vp, _l, _vp, _l, _i, _l, _vp, _vp]),
     "dftb_ensemble_workspace": (_sz, [ctypes.POINTER(EnsMolecule)]),
+    "dftb_ensemble_workspace_of_launch": (_sz, [ctypes.POINTER(EnsMolecule), _i]),
     "dftb_ensemble_solve": (_i, [_vp, _i, _d, _i, _vp]),
     "dftb_pair_features": (_i, [_vp, _vp, _vp, _vp, _vp, _l, _i, _vp, _vp]),
     "dftb_restricted_ab": (_i, [_vp, _vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _vp, _vp, _vp]),

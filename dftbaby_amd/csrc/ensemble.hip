@@ -492,7 +492,8 @@ __host__ __device__ static long ens_mmax(const EnsMolecule& m) {
   return a > b ? a : b;
 }
 
-__host__ __device__ static EnsLayout ens_layout(const EnsMolecule& m) {
+// nb: blocks per molecule of the launch; only TT, at the end, depends on it
+__host__ __device__ static EnsLayout ens_layout(const EnsMolecule& m, int nb) {
   EnsLayout L;
   const long N = (long)m.opad * m.vpad;
   const long rows = m.opad > m.vpad ? m.opad : m.vpad;
@@ -501,12 +502,12 @@ __host__ __device__ static EnsLayout ens_layout(const EnsMolecule& m) {
   // one TT per block while they stay within 256 MB
   L.tt = al256((size_t)m.nat * rows * m.vpad * 8);
   const size_t fit = L.tt > 0 ? ((size_t)1 << 28) / L.tt : 1;
-  L.slots = fit < 1 ? 1 : fit > ENS_BLOCKS ? ENS_BLOCKS : (int)fit;
+  L.slots = fit < 1 ? 1 : fit > (size_t)nb ? nb : (int)fit;
   size_t o = 0;
-  size_t* fields[] = {&L.TT, &L.X1, &L.X2, &L.tv, &L.gv, &L.Sq, &L.Sinv, &L.H, &L.Y2, &L.Z2, &L.P, &L.Tns, &L.eig,
+  size_t* fields[] = {&L.X1, &L.X2, &L.tv, &L.gv, &L.Sq, &L.Sinv, &L.H, &L.Y2, &L.Z2, &L.P, &L.Tns, &L.eig,
                       &L.Tbv, &L.Rb, &L.Lb, &L.R, &L.L, &L.PR, &L.ML, &L.W, &L.nrm, &L.w2, &L.G, &L.Li,
-                      &L.ref, &L.Qt, &L.v32, &L.keep, &L.ctl};
-  const size_t sizes[] = {L.tt * L.slots, (size_t)mm * N * 8, (size_t)mm * N * 8,
+                      &L.ref, &L.Qt, &L.v32, &L.keep, &L.ctl, &L.TT};
+  const size_t sizes[] = {(size_t)mm * N * 8, (size_t)mm * N * 8,
                           (size_t)mm * m.nat * 8, (size_t)mm * m.nat * 8, (size_t)cap * cap * 8,
                           (size_t)cap * cap * 8, (size_t)cap * cap * 8, (size_t)cap * cap * 8,
                           (size_t)cap * cap * 8, (size_t)cap * cap * 8, (size_t)cap * cap * 8,
@@ -514,7 +515,8 @@ __host__ __device__ static EnsLayout ens_layout(const EnsMolecule& m) {
                           (size_t)cap * k * 8, (size_t)k * N * 8, (size_t)k * N * 8, (size_t)k * N * 8,
                           (size_t)k * N * 8, (size_t)2 * k * N * 8, (size_t)2 * k * 8, (size_t)k * 8,
                           (size_t)mm * mm * 8, (size_t)mm * mm * 8, (size_t)mm * 8,
-                          (size_t)mm * N * 8, (size_t)mm * N * 4, (size_t)mm * 4, sizeof(EnsCtl)};
+                          (size_t)mm * N * 8, (size_t)mm * N * 4, (size_t)mm * 4, sizeof(EnsCtl),
+                          L.tt * L.slots};
   for (int i = 0; i < 30; ++i) {
     *fields[i] = o;
     o += al256(sizes[i]);
@@ -523,7 +525,19 @@ __host__ __device__ static EnsLayout ens_layout(const EnsMolecule& m) {
   return L;
 }
 
-extern "C" size_t dftb_ensemble_workspace(const EnsMolecule* m) { return ens_layout(*m).total; }
+// Blocks per molecule of a launch of nmol.  Helpers leave a quarter of the chip to other streams.
+// From ENS_GRID molecules on the leaders take the chip anyway, and helpers start as members end
+// (256 polyenes C8-C40: 2.25 s without helpers, 1.18 so).
+static int ens_blocks(int nmol) {
+  const int nb = nmol >= ENS_GRID ? ENS_BLOCKS : ENS_GRID / (nmol < 1 ? 1 : nmol);
+  return nb < 1 ? 1 : nb > ENS_BLOCKS ? ENS_BLOCKS : nb;
+}
+
+extern "C" size_t dftb_ensemble_workspace(const EnsMolecule* m) { return ens_layout(*m, ENS_BLOCKS).total; }
+
+extern "C" size_t dftb_ensemble_workspace_of_launch(const EnsMolecule* m, int nmol) {
+  return ens_layout(*m, ens_blocks(nmol)).total;
+}
 
 // --------------------------------------------------------------------------
 // matvec of m vectors V (FP64, [m][N]) -> outP = (A+B)V, outM = (A-B)V
@@ -605,9 +619,9 @@ __device__ void ens_matvec(EnsShare& sh, const EnsMolecule& Mo, char* ws, const 
 
 // helper number slot of a molecule: items until the leader ends
 template <typename T>
-__device__ void ens_help(const EnsMolecule& Mo, int slot, int* s_item) {
+__device__ void ens_help(const EnsMolecule& Mo, int slot, int nb, int* s_item) {
   char* ws = (char*)Mo.work;
-  const EnsLayout L = ens_layout(Mo);
+  const EnsLayout L = ens_layout(Mo, nb);
   EnsCtl* ctl = (EnsCtl*)(ws + L.ctl);
   if (slot >= L.slots) return;
   const unsigned long long mask = (1ull << ENS_ITEM_BITS) - 1;
@@ -786,8 +800,8 @@ template <typename T>
 __device__ void ens_davidson(const EnsMolecule& Mo, double conv, int maxiter, double* sh, double* sv, double* sp,
                              double* bnd, int* s_sel, double* stg, double* wl, int nb) {
   char* ws = (char*)Mo.work;
-  const EnsLayout L = ens_layout(Mo);
-  EnsShare es = {(EnsCtl*)(ws + L.ctl), 1, nb < L.slots ? nb : L.slots, s_sel + 2 * ENS_MAXK + 1, 0};
+  const EnsLayout L = ens_layout(Mo, nb);
+  EnsShare es = {(EnsCtl*)(ws + L.ctl), 1, L.slots, s_sel + 2 * ENS_MAXK + 1, 0};
   if (threadIdx.x == 0)
     __hip_atomic_store(&es.ctl->word, ENS_STARTED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // hands nothing over
   const long N = (long)Mo.opad * Mo.vpad;
@@ -1009,9 +1023,9 @@ __global__ __launch_bounds__(ENS_THREADS) void ensemble_kernel(const EnsMolecule
   const EnsMolecule& Mo = mols[mi];
   if (slot > 0) {
     if (Mo.precision == 1)
-      ens_help<float>(Mo, slot, s_sel);
+      ens_help<float>(Mo, slot, nb, s_sel);
     else
-      ens_help<double>(Mo, slot, s_sel);
+      ens_help<double>(Mo, slot, nb, s_sel);
   } else if (Mo.precision == 1)
     ens_davidson<float>(Mo, conv, maxiter, sh, sv, sp, bnd, s_sel, stg, wl, nb);
   else
@@ -1021,7 +1035,7 @@ __global__ __launch_bounds__(ENS_THREADS) void ensemble_kernel(const EnsMolecule
 __global__ void ensemble_begin_kernel(const EnsMolecule* __restrict__ mols, int nmol) {
   const int mi = blockIdx.x * blockDim.x + threadIdx.x;
   if (mi >= nmol) return;
-  EnsCtl* ctl = (EnsCtl*)((char*)mols[mi].work + ens_layout(mols[mi]).ctl);
+  EnsCtl* ctl = (EnsCtl*)((char*)mols[mi].work + ens_layout(mols[mi], 1).ctl);
   ctl->word = 0;
   ctl->done = 0;
   ctl->here = 0;
@@ -1029,11 +1043,7 @@ __global__ void ensemble_begin_kernel(const EnsMolecule* __restrict__ mols, int 
 
 extern "C" int dftb_ensemble_solve(const EnsMolecule* mols_dev, int nmol, double conv, int maxiter, void* stream) {
   if (!mols_dev || nmol <= 0 || maxiter <= 0) return DFTB_ERR_ARG;
-  // leaders come first in the grid; helpers leave a quarter of the chip to other streams.  From
-  // ENS_GRID molecules on the leaders take the chip anyway, and helpers start as members end
-  // (256 polyenes C8-C40: 2.25 s without helpers, 1.18 so).
-  int nb = nmol >= ENS_GRID ? ENS_BLOCKS : ENS_GRID / nmol;
-  nb = nb < 1 ? 1 : nb > ENS_BLOCKS ? ENS_BLOCKS : nb;
+  const int nb = ens_blocks(nmol);         // leaders come first in the grid
   hipLaunchKernelGGL(ensemble_begin_kernel, dim3((nmol + 63) / 64), dim3(64), 0, (hipStream_t)stream, mols_dev, nmol);
   DFTB_CHECK_LAUNCH();
   hipLaunchKernelGGL(ensemble_kernel, dim3(nmol * nb), dim3(ENS_THREADS), 0, (hipStream_t)stream, mols_dev, nmol, conv,

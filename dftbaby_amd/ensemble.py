@@ -102,7 +102,7 @@ def solve_operators(ops, nstates, conv=1.0e-6, maxiter=50, ifact=1, precision=0)
                 d.q32[j] = cp[key][0].data_ptr()
         d.guess = guess.data_ptr()
         d.bs, d.bp, d.bm, d.Mp, d.Mm = bs.data_ptr(), bp.data_ptr(), bm.data_ptr(), Mp.data_ptr(), Mm.data_ptr()
-        nb = _lib.load().dftb_ensemble_workspace(ctypes.byref(d))
+        nb = _lib.load().dftb_ensemble_workspace_of_launch(ctypes.byref(d), len(ops))
         work = torch.empty(int(nb), dtype=torch.uint8, device=dev)
         d.work = work.data_ptr()
         d.w, d.C, d.XmY, d.XpY, d.resid = w.data_ptr(), C.data_ptr(), XmY.data_ptr(), XpY.data_ptr(), resid.data_ptr()

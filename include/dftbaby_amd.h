@@ -310,12 +310,16 @@ typedef struct EnsMolecule {
   const long* guess;                    /* [nguess] flat padded indices */
   double *bs, *bp, *bm;                 /* [cap][opad*vpad] */
   double *Mp, *Mm;                      /* [cap][cap] */
-  void* work;                           /* dftb_ensemble_workspace() bytes */
+  void* work;                           /* dftb_ensemble_workspace[_of_launch]() bytes */
   double *w, *C, *XmY, *XpY, *resid;    /* outputs: [k], [k][N] x3, [k] */
   int* status;                          /* [3] */
 } EnsMolecule;
 
 size_t dftb_ensemble_workspace(const EnsMolecule* m);
+/* Bytes of EnsMolecule.work that a launch of nmol molecules uses: at most
+ * dftb_ensemble_workspace(), which serves a launch of any size, and without the
+ * expansion buffers of the blocks that this launch does not start. */
+size_t dftb_ensemble_workspace_of_launch(const EnsMolecule* m, int nmol);
 int dftb_ensemble_solve(const EnsMolecule* mols_dev, int nmol, double conv, int maxiter, void* stream);
 
 /* ---- learned initial space / preconditioner ---------------------------------

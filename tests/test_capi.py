@@ -105,3 +105,18 @@ def test_ensemble_workspace_of_an_empty_molecule(empty):
             "m.nat = m.nocc = m.nvirt = m.opad = m.vpad = m.k = m.cap = m.nguess = 8\n"
             "m.%s = 0\nassert _lib.load().dftb_ensemble_workspace(ctypes.byref(m)) > 0\n" % empty)
     assert subprocess.run([sys.executable, "-c", code], cwd=ROOT).returncode == 0
+
+
+@pytest.mark.parametrize("nmol,blocks", [(1, 8), (24, 8), (25, 7), (64, 3), (96, 2), (97, 1), (191, 1), (192, 8), (300, 8)])
+def test_ensemble_workspace_holds_the_buffers_of_its_launch(nmol, blocks):
+    """One expansion buffer (nat rows vpad doubles) per block that the launch starts for a molecule,
+    and no more; the size without a launch serves the most blocks."""
+    from dftbaby_amd import _lib
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("HIP library not built")
+    lib = _lib.load()
+    m = _lib.EnsMolecule()
+    m.nat, m.nocc, m.nvirt, m.opad, m.vpad, m.k, m.cap, m.nguess, m.lc = 100, 150, 130, 152, 136, 8, 300, 8, 1
+    buf = 100 * 152 * 136 * 8                       # a multiple of 256
+    most = lib.dftb_ensemble_workspace(ctypes.byref(m))
+    assert most - lib.dftb_ensemble_workspace_of_launch(ctypes.byref(m), nmol) == (8 - blocks) * buf
