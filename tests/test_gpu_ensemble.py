@@ -54,3 +54,22 @@ def test_ensemble_batch_size_does_not_show(copies, precision, conv, tol):
         for w, xpy in zip(res.Omega, res.XpY):
             assert np.abs(w - ref_w).max() < tol, (w, ref_w)
             assert np.array_equal(w, alone.Omega[0]) and np.array_equal(xpy, alone.XpY[0])
+
+
+@pytest.mark.parametrize("count", [150, 192, 300])
+def test_large_ensembles(count):
+    """Launches without helpers (150), with helpers that start as members end (192) and with more
+    members than CUs (300): the bits of each member alone, and energies within the bound above."""
+    from conftest import progress
+    from dftbaby_amd.ensemble import build_operators, solve_operators
+    kinds = [ground_state("C8H10", 1, 0.05, 7), ground_state("C12H14", 1, 0.05, 8), ground_state("C8H10", 1, 0.05, 9)]
+    which = [1 if i % 50 == 7 else 2 * (i % 2) for i in range(count)]
+    alone = [solve_operators(build_operators([gs]), 5, conv=1e-6, maxiter=100, precision=1) for gs in kinds]
+    for gs, one in zip(kinds, alone):
+        assert np.abs(one.Omega[0] - _oracle(gs, 5, 1e-8)[0]).max() < 1e-6
+    ops = build_operators([kinds[i] for i in which])
+    progress("%d operators" % count)
+    res = solve_operators(ops, 5, conv=1e-6, maxiter=100, precision=1)
+    for i, w, xpy, n in zip(which, res.Omega, res.XpY, res.iterations):
+        assert n == alone[i].iterations[0]
+        assert np.array_equal(w, alone[i].Omega[0]) and np.array_equal(xpy, alone[i].XpY[0])
