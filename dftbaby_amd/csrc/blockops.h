@@ -360,10 +360,11 @@ __device__ void cluster_wave(int l, int nev, int m0, int m1, const double* __res
 // Householder steps j0 <= j < j1 in one workgroup.  X(r, c) = X[r * ldx + c] holds the rows and
 // columns j0, .. l - 1 of the matrix, in LDS or in global memory; reflector j goes to row j of W
 // behind the diagonal (never read again by the reduction), where the back-transformation reads it
-// coalesced.  A wave takes RB rows and CB chunks of 64 columns at a time: a load's latency, not its
-// bandwidth, bounds a step.
+// coalesced.  X may be W itself: row j is then written through X in step j - 1 and through W in
+// step j, with barriers between.  A wave takes RB rows and CB chunks of 64 columns at a time: a
+// load's latency, not its bandwidth, bounds a step.
 template <int RB, int CB, typename P>
-__device__ __forceinline__ void hh_block_steps(P X, int ldx, int j0, int j1, int l, double* __restrict__ W,
+__device__ __forceinline__ void hh_block_steps(P X, int ldx, int j0, int j1, int l, double* W,
                                                double* __restrict__ d, double* __restrict__ e,
                                                double* __restrict__ tau, lds_f64* sv, lds_f64* sp, double* sh) {
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nw = blockDim.x >> 6;

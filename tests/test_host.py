@@ -24,3 +24,15 @@ def test_zvector_solver_needs_the_gpu_operator():
     from dftbaby_amd import Solver
     with pytest.raises(TypeError):
         Solver.Krylov_solver_Zvector(lambda x: x, np.ones((2, 3)), np.ones((2, 3, 1)), None)
+
+
+def test_householder_steps_promise_no_separate_matrix():
+    """syevx_block runs the Householder steps on W itself (X = W) for matrices beyond the LDS, so the
+    function that takes both must not declare W free of aliases."""
+    import os
+    import re
+    from conftest import ROOT
+    src = open(os.path.join(ROOT, "dftbaby_amd", "csrc", "blockops.h")).read()
+    assert re.search(r"hh_block_steps<\d+, \d+>\(W, [^;]*, W,", src)
+    params = re.search(r"void hh_block_steps\(([^)]*)\)", src).group(1)
+    assert re.search(r"double\s*\*\s*W\b", params) and not re.search(r"__restrict__\s+[XW]\b", params)
