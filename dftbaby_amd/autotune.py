@@ -2,8 +2,9 @@
 
 For one operator and precision it times candidate launch shapes with HIP events
 on the launch stream and keeps the fastest in ``op.tuning[precision]``, which
-the operator passes to every later matvec (CasidaOperator fields ``atom_chunk``,
-``tile_expand``, ``tile_contract``):
+the operator passes to later matvecs (CasidaOperator fields ``atom_chunk``,
+``tile_expand``, ``tile_contract``; the tiles for blocks of at least half as many
+vectors as they were measured on, smaller ones take the library's choice by size):
 
 * AO-basis exchange in BF16x3 (the default exchange of the mixed modes): the
   pipelined tile of the first two GEMMs of each exchange chain (B1 and the
@@ -14,7 +15,7 @@ the operator passes to every later matvec (CasidaOperator fields ``atom_chunk``,
   timed on the exchange restricted to an atom slice (``atom_limit``) and
   normalised per atom.
 
-Results are cached per (precision, exchange, shape bucket) in a JSON file so
+Results are cached per (kernel generation, precision, exchange, shape bucket) in a JSON file so
 later operators of a similar size reuse them without measuring.
 """
 import json
@@ -26,9 +27,12 @@ import torch
 CACHE = os.path.join(os.path.expanduser("~"), ".cache", "dftbaby_amd", "tuning.json")
 
 
+KERNELS = 2      # counts up when other kernels or tile rules make earlier measurements void
+
+
 def _bucket(op, precision):
     b = lambda x: int(2 ** np.round(np.log2(max(x, 1))))
-    return "p%d_%s_nat%d_o%d_v%d" % (precision, op.exchange, b(op.nat), b(op.nocc), b(op.nvirt))
+    return "k%d_p%d_%s_nat%d_o%d_v%d" % (KERNELS, precision, op.exchange, b(op.nat), b(op.nocc), b(op.nvirt))
 
 
 def _time(fn, reps):
@@ -76,7 +80,7 @@ def _load(path):
 def autotune(op, precision, nvec=40, atom_chunks=(8, 16, 32, 64), tiles=(64, 128), reps=2, cache=CACHE,
              use_cache=True, log=None):
     """Pick the launch shapes of op's matvec at this precision (0 fp64, 1 fp32,
-    2 bf16x3); store them in op.tuning (used by every later matvec) and the cache."""
+    2 bf16x3); store them in op.tuning (used by later matvecs) and the cache."""
     key = _bucket(op, precision)
     table = _load(cache) if use_cache else {}
     if use_cache and key in table:

@@ -253,8 +253,9 @@ static int ao_gemm(int prec, const void* A, const void* A2, long lda, const void
                    long sB, int btrans, void* C, void* C2, long ldc, long sC, int M, int N, int K, int batch,
                    double alpha, bool final, const CasidaOperator* op, bool had, hipStream_t st, int tile = 0) {
   GemmArgs g = gemm_args_default();
-  // a tuned pipelined tile (256: 256 x 128, 512: 256 x 256) applies where the
-  // automatic choice is the pipelined kernel too
+  // a tuned pipelined tile (256: 256 x 128, 512: 256 x 256) applies to products of at least one
+  // such tile, whatever the rule by size would take; the caller gives it for blocks of about the
+  // size it was measured on
   g.tile = (prec == 2 && (tile == 256 || tile == 512) && M >= 256 && N >= 128 && K >= 128) ? tile : 0;
   g.in_type = prec == 0 ? GEMM_IN_F64 : (prec == 1 ? GEMM_IN_F32 : GEMM_IN_BF16X3);
   g.out_type = final ? GEMM_OUT_F64 : (prec == 0 ? GEMM_OUT_F64 : (prec == 1 ? GEMM_OUT_F32 : GEMM_OUT_BF16PAIR));
