@@ -56,7 +56,10 @@ __global__ __launch_bounds__(EIG_THREADS) void syevx_kernel(const double* __rest
 // back-transformation.  Entries (r, c) and (c, r) agree to rounding (the update term's two
 // products are rounded differently), so row j + 1 is column j + 1 to rounding.
 #define HH_THREADS 512
-#define HH_PRE 10   // row entries per lane loaded ahead (rows up to 640)
+// row entries per lane loaded ahead, 64 HH_PRE of a row; longer rows load the rest in the loop.
+// 10, 13 and 16 differ by less than 3% (l = 400: 3.36, 3.38, 3.43 ms of dftb_syevx; 800: 7.43, 7.40,
+// 7.54; 1500: 18.7, 18.4, 18.2)
+#define HH_PRE 10
 
 __global__ __launch_bounds__(256) void sym_copy_kernel(const double* __restrict__ A, int l, int ld, double* __restrict__ W) {
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < (long)l * l; i += (long)gridDim.x * blockDim.x) {
@@ -232,7 +235,7 @@ __global__ __launch_bounds__(HH_THREADS) void hh_step_kernel(double* __restrict_
   hh_step_body(W, l, j, col, coln, P, Pn, d, e, tau, hv0, blockIdx.x, gridDim.x, sv, sw, sn, sh);
 }
 
-// Steps j0 .. l - 3 of hh_step in one workgroup with the trailing block in LDS (n0 = l - j0
+// Steps j0 .. l - 3 of hh_step in one workgroup with the trailing block in LDS (n0 = l - j0 - 1
 // <= HH_LDS_N rows; same operations in the same order, so the results are those of the
 // launches it replaces).  A launch per column costs 5.6 us at any size below ~200; here a
 // column of the last 136 takes 3.6 us.  On entry col / P are step j0's, as for hh_step;

@@ -8,10 +8,15 @@
 // rates (2.5 PFLOP/s bf16 vs 157 TFLOP/s fp32).
 //
 // Measured limits on gfx950 (register-only loops): v_mfma_f32_16x16x32_bf16
-// sustains about 1.46 PFLOP/s, v_mfma_f32_32x32x16_bf16 about 2.46 PFLOP/s.  The
-// pipelined kernel below is bound by its global->LDS feed (with the DMA removed
-// the same loop reaches about 74% of 2.5 PFLOP/s, with the MFMAs removed it takes
-// as long as the full kernel), which is why its tile order is grouped per XCD.
+// sustains about 1.46 PFLOP/s, v_mfma_f32_32x32x16_bf16 about 2.46 PFLOP/s.  With
+// 256 x 128 tiles the pipelined kernel below was held by its global->LDS feed (with
+// the DMA removed the same loop reached 62-74% of 2.5 PFLOP/s, with the MFMAs removed
+// it took as long), which is why its tile order is grouped per XCD.  With 256 x 256
+// tiles the launches without a transposed copy reach 1.16 PFLOP/s, MFMA busy 58% of
+// the cycles; fewer LDS and DMA waits (four waves, reads under the MFMAs) and L2
+// prefetch left the cycles as they were, so neither LDS nor L2 holds that loop, and
+// what does is not settled.  With the copy (39 stages per tile) it is 0.82: the
+// epilogue, about 60 us of each round, runs under no MFMAs.
 //
 // Form: C = A B^T ("NT"): A[m][k] and B[n][k] both K-contiguous, so every lane
 // loads its 8 consecutive k values for one row with a single 16-byte LDS read,
@@ -735,9 +740,8 @@ int gemm_bf16x3_launch(const GemmArgs& p, hipStream_t st) {
     dim3 grid(ceil_div(p.N, bn), ceil_div(p.M, P_BM), p.batch * p.ksplit);
     GemmTimer tm;
     tm.begin(st);
-    // 16x16x32 by default: the kernel is bound by its global->LDS feed, where the
-    // 16x16 form measured 2-4% faster (256 x 128 tiles); DFTB_BF3_M32=1 selects the
-    // 32x32x16 form
+    // 16x16x32 by default: measured 2-4% faster with 256 x 128 tiles and 1-8% with
+    // 256 x 256 ones; DFTB_BF3_M32=1 selects the 32x32x16 form
     static const int m32_env = getenv("DFTB_BF3_M32") ? atoi(getenv("DFTB_BF3_M32")) : 0;
     const int m32 = m32_env;
     const dim3 block(DFTB_BF3_WAVES * 64);
